@@ -292,6 +292,70 @@ def test_attention_prefill_matches_oracle_per_token(dev, layer_index, first, tok
         b.free()
 
 
+# One to four chunks of 64 positions (the second group of waves takes every other one, none
+# of a single chunk), blocks that straddle a chunk, one token past a block; some sinks
+# -infinity, so that a chunk masked as a whole has no maximum of its own.
+@pytest.mark.parametrize("layer_index", [0, 1])
+@pytest.mark.parametrize("first,tokens", [(0, 1), (0, 17), (56, 24), (63, 2), (120, 33), (200, 50)])
+def test_attention_prefill_chunk_edges(dev, layer_index, first, tokens):
+    capacity = first + tokens
+    q = O.synth_normal(61, first, tokens * 4096, sigma=2.0)
+    k = O.synth_normal(62, first, capacity * 512, sigma=2.0)
+    v = O.synth_normal(63, first, capacity * 512)
+    sinks = O.synth_normal(64, 0, 64, sigma=2.0)
+    sinks[::5] = -np.inf
+    check_attention_prefill(dev, q, k, v, sinks, layer_index, first, tokens, capacity)
+
+
+# Values the three bf16 planes do not take (K of 2^60 and more, V of 2^100 and more,
+# infinities; a query of 2^60) next to ordinary ones: the chunks that hold them, and no
+# others, run on f32 MFMA.  Finite outputs within the usual bar, the others where the
+# oracle has them.
+@pytest.mark.parametrize("layer_index", [0, 1])
+@pytest.mark.parametrize("kind", ["k_large", "k_inf", "v_large", "v_inf", "q_large"])
+def test_attention_prefill_wide_values(dev, layer_index, kind):
+    first, tokens = 90, 40
+    capacity = first + tokens
+    q = O.synth_normal(71, 0, tokens * 4096, sigma=2.0)
+    k = O.synth_normal(72, 0, capacity * 512, sigma=2.0)
+    v = O.synth_normal(73, 0, capacity * 512)
+    sinks = O.synth_normal(74, 0, 64, sigma=2.0)
+    k2, v2, q2 = k.reshape(capacity, 8, 64), v.reshape(capacity, 8, 64), q.reshape(tokens, 64, 64)
+    if kind == "k_large":
+        k2[100, 3] *= np.float32(2.0**60)
+    elif kind == "k_inf":
+        k2[100, 3, 5] = np.inf
+    elif kind == "v_large":
+        v2[70, 2] *= np.float32(2.0**101)
+    elif kind == "v_inf":
+        v2[70, 2, 9] = -np.inf
+    else:
+        q2[5, 17] *= np.float32(2.0**60)
+    check_attention_prefill(dev, q, k, v, sinks, layer_index, first, tokens, capacity)
+
+
+def check_attention_prefill(dev, q, k, v, sinks, layer_index, first, tokens, capacity):
+    bufs = [dev.upload(a) for a in (q, k, v, sinks)]
+    out = dev.alloc(tokens * 4096 * 4)
+    dev.attention_prefill(*bufs, first, tokens, capacity, layer_index, out)
+    got = out.download(np.float32).reshape(tokens, 64, 64)
+    ref = np.empty(4096, np.float32)
+    scores = np.empty(capacity, np.float32)
+    for t in range(tokens):
+        O.lib.orc_attention(np.ascontiguousarray(q[t * 4096:(t + 1) * 4096]), k, v, sinks, layer_index, first + t,
+                            ref, scores)
+        r = ref.reshape(64, 64)
+        fine = np.isfinite(r)
+        assert np.array_equal(fine, np.isfinite(got[t])) and np.array_equal(np.isnan(r), np.isnan(got[t]))
+        assert np.array_equal(r[np.isinf(r)], got[t][np.isinf(r)])
+        for h in range(64):  # heads apart: their magnitudes differ by up to 2^100
+            f = fine[h]
+            err = np.linalg.norm((got[t, h][f] - r[h][f]).astype(np.float64))
+            assert err <= TOL * np.linalg.norm(r[h][f].astype(np.float64)), (t, h)
+    for b in bufs + [out]:
+        b.free()
+
+
 def test_attention_prefill_rejects_bad_shapes(dev):
     buf = dev.alloc(4096 * 4)
     cache = dev.alloc(64 * 512 * 4)

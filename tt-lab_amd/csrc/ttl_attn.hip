@@ -343,185 +343,528 @@ __global__ __launch_bounds__(kWinThreads) void attn_window_kernel(const float *_
     }
 }
 
-// Prefill: attention of a run of tokens on f32 MFMA, v_mfma_f32_16x16x4_f32 (D 16x16
-// += A 16x4 B 4x16; lane l holds A[l%16][l/16] and B[l/16][l%16] and receives D rows
-// 4(l/16)..+3 of column l%16).  One workgroup per (kv head, 16 consecutive tokens):
-// the 8 query heads of the group times 16 tokens are 128 queries, in tiles of 16, two
-// tiles per wave.  The union of the block's spans streams through LDS in chunks of 64
-// positions, each K/V row loaded once per workgroup.  Per chunk and query tile:
-//  - S^T (positions x queries) = K Q^T: A is 16 K rows from LDS, B the tile's queries,
-//    held in registers for the whole launch; K step (s, j) covers dims 16s + 4k + j for
-//    lane group k, so each lane reads its K operands as float4;
-//  - an online softmax per query (a column of S^T: the lane's 4 rows of each position
-//    tile and the 4 lanes of its column).  m starts at the sink and l at
-//    exp(sink - sink) = 1, so the sink takes part in the max and the denominator
-//    (model.cpp:270-281); per chunk m' = max(m, scores), and l and O are rescaled by
-//    exp(m - m');
-//  - O^T (dims x queries) += V^T P^T: K step j of position tile p takes positions
-//    16p + 4k + j for lane group k, which is row j of the lane's own S^T tile, so the
-//    probabilities never leave their registers; A reads V rows from LDS.
+// Prefill: attention of a run of tokens on bf16 MFMA, every f32 operand as three bf16
+// planes.  One workgroup per (kv head, 16 consecutive tokens): the 8 query heads of the
+// group times 16 tokens are 128 queries, in tiles of 16, two tiles per wave of a group of
+// four waves.  Two such groups share the workgroup and take the chunks of 64 positions in
+// turn (group 0 the first, third, ..., group 1 the others), each with an online softmax
+// of its own; group 0 merges the two at the end.  Per chunk and query tile:
+//  - S^T (positions x queries) = K Q^T, then an online softmax per query (a column of S^T:
+//    the lane's 4 rows of each position tile and the 4 lanes of its column).  m starts at
+//    the sink and l (group 0) at exp(sink - sink) = 1, so the sink takes part in the max
+//    and the denominator (model.cpp:270-281); per chunk m' = max(m, scores), and l and O
+//    are rescaled by exp(m - m');
+//  - O^T (dims x queries) += V^T P^T.
 // The output is O / l.
+//
+// v_mfma_f32_16x16x32_bf16 (D = A B + C): lane (n, g) = (l % 16, l / 16) holds 8 bf16 of
+// A row n and of B column n for 8 of the 32 K indices, the same for A and B, and receives
+// D rows 4g..4g+3 of column n.  In the first product lane group g takes dims 8g..8g+7 of
+// each half of the head.  In the second, K step h covers position tiles 2h and 2h + 1, and
+// lane group g takes positions 16 (2h) + 4g + i and 16 (2h + 1) + 4g + i, i = 0..3: the
+// rows of the lane's own S^T tiles, so the probabilities never leave their registers; V is
+// staged transposed, with the positions of a dim in that order.
+//
+// Numerics: x = x0 + x1 + x2, each plane the remainder rounded to bf16, holds every f32 to
+// its last bit or 2^-25 of it; the products x0 y0, x0 y1, x1 y0, x1 y1, x0 y2, x2 y0 are
+// exact in f32 and the three left out are at most 2^-24 of |x y|, as much as f32 rounds
+// the product itself.  Relative error against 64 bits, 512 tokens at 1536 (a sliding and a
+// full layer): 3.9e-7 on f32 MFMA, 2.4e-7 this way.  The planes assume magnitudes whose
+// sums stay finite: a chunk with a K of 2^60 or more, a V of 2^100 or more, an infinity or
+// a NaN, and every chunk of a block with such a query, takes f32 MFMA (attn_chunk_f32).
+//
+// What bounds it: on v_mfma_f32_16x16x4_f32 a chunk's two products of a wave take 256
+// instructions of 32 cycles; six bf16 products take 192 of 16, and the second group puts a
+// second wave on each SIMD, whose softmax and splitting partly overlap the other's MFMAs.
+// Matrix cores about 40% busy, the VALU (splits, softmax, addresses) as much.  512 tokens
+// at 1536: 237 us for a sliding and a full layer on f32 MFMA with one group, 111 us now (on
+// the way: planes 134, scores in units of log 2 125, LDS in fragment order and a barrier
+// per group 113).
 constexpr int kPfTokens = 16;
-constexpr int kPfQueries = kPfTokens * kGroup;                // 128
-constexpr int kPfThreads = 256;
-constexpr int kPfTiles = kPfQueries / 16 / (kPfThreads / 64);  // query tiles per wave: 2
+constexpr int kPfQueries = kPfTokens * kGroup;                   // 128
+constexpr int kPfGroups = 2;                                     // groups of four waves
+constexpr int kPfGroupThreads = 256;
+constexpr int kPfThreads = kPfGroups * kPfGroupThreads;
+constexpr int kPfTiles = kPfQueries / 16 / (kPfGroupThreads / 64);  // query tiles per wave: 2
+constexpr int kPfPlanes = 3;
+constexpr int kPfPlane = kChunk * kHead;  // bf16 of one staged plane, in fragment order [fragment][lane][8]
+
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 __device__ inline mf::f32x4 mfma_f32(float a, float b, const mf::f32x4 &c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-__global__ __launch_bounds__(kPfThreads) void attn_prefill_kernel(const float *__restrict__ q,
-                                                                  const float *__restrict__ k_cache,
-                                                                  const float *__restrict__ v_cache,
-                                                                  const float *__restrict__ sinks, uint32_t first,
-                                                                  uint32_t tokens, uint32_t layer_index,
-                                                                  float *__restrict__ out) {
+// Two f32 as three planes of two packed bf16 each (the first value in the low half).
+__device__ __attribute__((always_inline)) inline void split3(float a, float b, uint32_t (&out)[kPfPlanes]) {
+#pragma unroll
+    for (int p = 0; p < kPfPlanes; ++p) {
+        const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, mf::bf16x2));
+        out[p] = w;
+        a -= __uint_as_float(w << 16);
+        b -= __uint_as_float(w & 0xffff0000u);
+    }
+}
+
+// The planes of (a, b) x log2(e) / 8, the product carried past f32 into the last plane.
+__device__ __attribute__((always_inline)) inline void split3_scaled(float a, float b, uint32_t (&out)[kPfPlanes]) {
+#pragma clang fp contract(off)  // ah and bh are the rounded products
+    constexpr float c = 0x1.715476p-3f, c_lo = 0x1.4ae0cp-29f;
+    const float ah = a * c, bh = b * c;
+    const float al = fmaf(a, c_lo, fmaf(a, c, -ah)), bl = fmaf(b, c_lo, fmaf(b, c, -bh));
+    float ra = ah, rb = bh;
+#pragma unroll
+    for (int p = 0; p < kPfPlanes; ++p) {
+        const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{ra, rb}, mf::bf16x2));
+        out[p] = w;
+        ra -= __uint_as_float(w << 16);
+        rb -= __uint_as_float(w & 0xffff0000u);
+        if (p == kPfPlanes - 2) {
+            ra += al;
+            rb += bl;
+        }
+    }
+}
+
+// The larger magnitudes of two packed pairs of bf16 (as bit patterns, so infinities and
+// NaNs are the largest), and whether one of a pair is 2^E or more.
+__device__ inline uint32_t pair_max(uint32_t acc, uint32_t w) {
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, acc),
+                                                                  __builtin_bit_cast(u16x2, w & 0x7fff7fffu)));
+}
+template <int E>
+__device__ inline bool at_least(uint32_t pair) {
+    constexpr uint32_t bits = uint32_t(E + 127) << 7;
+    return (pair & 0xffffu) >= bits || (pair >> 16) >= bits;
+}
+constexpr int kPfKMax = 60, kPfVMax = 100;  // and 2^60 for the queries
+
+// Scores and their maxima are kept in units of log 2 (times log2 e), so a probability is
+// one v_exp_f32 (1 ulp); the factor goes into the queries, carried past f32.
+constexpr float kLog2e = 0x1.715476p+0f, kLog2eLo = 0x1.4ae0cp-26f;  // log2 e = their sum
+constexpr float kPfMasked = -3.0e38f;  // a masked score: exp2 of its distance to any maximum is zero
+
+// The online softmax state of a wave's queries.
+struct PfState {
+    float m[kPfTiles], l[kPfTiles];
+    mf::f32x4 o[kPfTiles][4];  // O^T tiles: dims 16M + 4g + i of the query
+};
+
+// The running maximum and rescaling of one query tile for a chunk whose largest score of
+// the lane is cmax.  (A sink of -infinity and a chunk masked as a whole: the maximum is
+// kPfMasked or -infinity, and the first real score's rescaling takes what was summed to
+// zero.)
+__device__ __attribute__((always_inline)) inline float pf_rescale(PfState &st, int qi, float cmax) {
+    cmax = fmaxf(cmax, __shfl_xor(cmax, 16));
+    cmax = fmaxf(cmax, __shfl_xor(cmax, 32));
+    const float m2 = fmaxf(st.m[qi], cmax);
+    const float scale = m2 == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(st.m[qi] - m2);
+    st.l[qi] *= scale;
+    st.m[qi] = m2;
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            st.o[qi][mt][i] *= scale;
+        }
+    }
+    return m2;
+}
+
+// One chunk on f32 MFMA, operands straight from global memory: K step (s, j) of the scores
+// covers dims 16s + 4k + j for lane group k; K step j of position tile p of the second
+// product takes positions 16p + 4k + j.
+struct PfQueries {
+    uint32_t row[kPfTiles], first[kPfTiles], pos[kPfTiles];
+};
+__device__ __attribute__((noinline)) void attn_chunk_f32(const float *q, const float *k_cache, const float *v_cache,
+                                                         uint32_t kvh, uint32_t c0, uint32_t hi, const PfQueries &qs,
+                                                         uint32_t n, uint32_t g, PfState &st) {
+#pragma clang fp contract(off)  // s x log2 e rounded alike in the maximum and in the distance to it
     using mf::f32x4;
-    __shared__ __attribute__((aligned(16))) float ks[kChunk * kRowStride];
-    __shared__ __attribute__((aligned(16))) float vs[kChunk * kRowStride];
-    const uint32_t t = threadIdx.x, wave = t / 64, lane = t % 64, n = lane % 16, g = lane / 16;
+#pragma unroll 1
+    for (int qi = 0; qi < kPfTiles; ++qi) {
+        const float *qr = q + size_t(qs.row[qi]) * kHead;
+        f32x4 sc[4];
+        float cmax = -INFINITY;
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            sc[p] = f32x4{0.f, 0.f, 0.f, 0.f};
+            const size_t row = (size_t(min(c0 + 16 * p + n, hi)) * kKvHeads + kvh) * kHead;
+            for (int s4 = 0; s4 < 4; ++s4) {
+                const float4 a = *reinterpret_cast<const float4 *>(k_cache + row + 16 * s4 + 4 * g);
+                const float4 b = *reinterpret_cast<const float4 *>(qr + 16 * s4 + 4 * g);
+                sc[p] = mfma_f32(a.x, b.x, sc[p]);
+                sc[p] = mfma_f32(a.y, b.y, sc[p]);
+                sc[p] = mfma_f32(a.z, b.z, sc[p]);
+                sc[p] = mfma_f32(a.w, b.w, sc[p]);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t at = c0 + 16 * p + 4 * g + i;
+                const float s = at >= qs.first[qi] && at <= qs.pos[qi] ? sc[p][i] * 0.125f : -INFINITY;
+                sc[p][i] = s;
+                cmax = fmaxf(cmax, s * kLog2e);
+            }
+        }
+        const float m2 = pf_rescale(st, qi, cmax);
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float s = sc[p][i];
+                // the product's low part, for scores small enough that it says something
+                const float hi2 = s * kLog2e, lo2 = fmaf(s, kLog2eLo, fmaf(s, kLog2e, -hi2));
+                const float x = (hi2 - m2) + (fabsf(s) < 0x1p14f ? lo2 : 0.0f);
+                sc[p][i] = s == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(x);
+                st.l[qi] += sc[p][i];
+            }
+        }
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const size_t row = (size_t(min(c0 + 16 * p + 4 * g + j, hi)) * kKvHeads + kvh) * kHead;
+#pragma unroll
+                for (int mt = 0; mt < 4; ++mt) {
+                    st.o[qi][mt] = mfma_f32(v_cache[row + 16 * mt + n], sc[p][j], st.o[qi][mt]);
+                }
+            }
+        }
+    }
+}
+
+// A barrier of one group's four waves (every wave of the group arrives, each time): a count
+// in LDS that only grows, `target` its value once all have arrived.  LDS operations of a
+// wave are done in order, so an arrival follows the wave's earlier LDS accesses.  With
+// s_barrier the two groups ran in step, both on the matrix cores and then both on the VALU.
+__device__ __attribute__((always_inline)) inline void group_sync(uint32_t *count, uint32_t target, uint32_t lane) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (lane == 0) {
+        __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    while (uint32_t(__builtin_amdgcn_readfirstlane(
+               __hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP))) < target) {
+    }
+    asm volatile("" ::: "memory");
+}
+
+__global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2))) void attn_prefill_kernel(
+    const float *__restrict__ q, const float *__restrict__ k_cache, const float *__restrict__ v_cache,
+    const float *__restrict__ sinks, uint32_t first, uint32_t tokens, uint32_t layer_index,
+    float *__restrict__ out) {
+    using mf::bf16x8;
+    using mf::f32x4;
+    // per group: K planes in fragments (position tile, half of the head), V planes in
+    // fragments (dim tile, K step)
+    __shared__ __attribute__((aligned(16))) uint16_t kv[kPfGroups][2][kPfPlanes][kPfPlane];
+    __shared__ uint32_t odd[kPfGroups][2];  // a chunk for the f32 path, by iteration parity
+    __shared__ uint32_t odd_query;
+    __shared__ uint32_t arrived[kPfGroups];
+    const uint32_t t = threadIdx.x % kPfGroupThreads, grp = threadIdx.x / kPfGroupThreads;
+    const uint32_t wave = t / 64, lane = t % 64, n = lane % 16, g = lane / 16;
     const uint32_t kvh = blockIdx.y, block0 = blockIdx.x * kPfTokens;
     const uint32_t last_local = min(block0 + kPfTokens, tokens) - 1;
     // the block's positions: from the first token's span start to the last token
     const uint32_t lo = span_of(first + block0, layer_index).first;
     const uint32_t hi = first + last_local;
+    const uint32_t start = lo - lo % kChunk;
+    const uint32_t chunks = (hi - start) / kChunk + 1;
+    const uint32_t rounds = (chunks + kPfGroups - 1 - grp) / kPfGroups;  // this group's chunks
 
-    // this lane's query (column n) of each of the wave's tiles
-    float qv[kPfTiles][16];  // [4s + j] = Q[dim 16s + 4g + j]
-    uint32_t qpos[kPfTiles], qfirst[kPfTiles], qlocal[kPfTiles], qhead[kPfTiles];
-    float m[kPfTiles], l[kPfTiles];
-    f32x4 o[kPfTiles][4];  // O^T tiles: dims 16M + 4g + i of the query
+    // staging, so that the LDS stores spread over the banks as the fragment reads do: of K,
+    // position n of each tile and dims 4 dq..+3; of V, dim `lane` of the wave's position tile
+    const uint32_t dq = 4 * wave + g;
+    float4 kr[4];
+    float vr[16];
+    auto request = [&](uint32_t round) __attribute__((always_inline)) {
+        // positions past the block's last re-read it
+        const uint32_t c0 = start + (round * kPfGroups + grp) * kChunk;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const uint32_t kp = min(c0 + 16 * k + n, hi);
+            kr[k] = *reinterpret_cast<const float4 *>(k_cache + (size_t(kp) * kKvHeads + kvh) * kHead + 4 * dq);
+        }
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            const uint32_t vp = min(c0 + 16 * wave + k, hi);
+            vr[k] = v_cache[(size_t(vp) * kKvHeads + kvh) * kHead + lane];
+        }
+    };
+    request(0);
+
+    // this lane's query (column n) of each of the wave's tiles, as B fragments of K step s
+    uint32_t qp[kPfTiles][2][kPfPlanes][4];
+    uint32_t qpos[kPfTiles], qfirst[kPfTiles], qrow[kPfTiles];
+    bool live[kPfTiles];
+    PfState st;
+    uint32_t bad_query = 0;
 #pragma unroll
     for (int qi = 0; qi < kPfTiles; ++qi) {
         const uint32_t query = (wave * kPfTiles + qi) * 16 + n;
-        qlocal[qi] = block0 + query / kGroup;
-        qhead[qi] = kvh * kGroup + query % kGroup;
-        const uint32_t lc = min(qlocal[qi], last_local);  // past the last token: a stand-in, not written
+        const uint32_t local = block0 + query / kGroup, head = kvh * kGroup + query % kGroup;
+        live[qi] = local < tokens;
+        const uint32_t lc = min(local, last_local);  // past the last token: a stand-in, not written
         qpos[qi] = first + lc;
         qfirst[qi] = span_of(qpos[qi], layer_index).first;
-        const float4 *q4 = reinterpret_cast<const float4 *>(q + (size_t(lc) * kQHeads + qhead[qi]) * kHead);
+        qrow[qi] = lc * kQHeads + head;
+        const float4 *q4 = reinterpret_cast<const float4 *>(q + size_t(qrow[qi]) * kHead);
 #pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4) {
-            const float4 v = q4[4 * s4 + g];
-            qv[qi][4 * s4] = v.x;
-            qv[qi][4 * s4 + 1] = v.y;
-            qv[qi][4 * s4 + 2] = v.z;
-            qv[qi][4 * s4 + 3] = v.w;
+        for (int s = 0; s < 2; ++s) {
+            const float4 a = q4[8 * s + 2 * g], b = q4[8 * s + 2 * g + 1];
+            const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                uint32_t w[kPfPlanes];
+                split3_scaled(v[2 * e], v[2 * e + 1], w);
+                bad_query = pair_max(bad_query, w[0]);
+#pragma unroll
+                for (int p = 0; p < kPfPlanes; ++p) {
+                    qp[qi][s][p][e] = w[p];
+                }
+            }
         }
-        m[qi] = sinks[qhead[qi]];
-        l[qi] = g == 0 ? 1.0f : 0.0f;  // the sink's exp(sink - m), counted once per column
+        st.m[qi] = sinks[head] * kLog2e;
+        st.l[qi] = g == 0 && grp == 0 ? 1.0f : 0.0f;  // the sink's exp(sink - m), counted once per column
 #pragma unroll
         for (int mt = 0; mt < 4; ++mt) {
-            o[qi][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+            st.o[qi][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
     }
+    if (threadIdx.x < 2 * kPfGroups) {
+        (&odd[0][0])[threadIdx.x] = 0;
+    }
+    if (threadIdx.x < kPfGroups) {
+        arrived[threadIdx.x] = 0;
+    }
+    if (threadIdx.x == 0) {
+        odd_query = 0;
+    }
+    __syncthreads();
+    if (at_least<kPfKMax>(bad_query)) {
+        odd_query = 1;
+    }
+    __syncthreads();
 
-    constexpr int kPer = kChunk * (kHead / 4) / kPfThreads;  // 4 float4 of K and of V per thread
-    for (uint32_t c0 = lo - lo % kChunk; c0 <= hi; c0 += kChunk) {
-        __syncthreads();  // the previous chunk's reads are done
+    uint16_t *const ks = kv[grp][0][0], *const vs = kv[grp][1][0];
+    const auto frag = [&](const uint16_t *base, int plane, int f) __attribute__((always_inline)) {
+        return *reinterpret_cast<const bf16x8 *>(base + plane * kPfPlane + f * 512 + lane * 8);
+    };
+    const auto q_frag = [&](int qi, int s, int p) __attribute__((always_inline)) {
+        return __builtin_bit_cast(bf16x8, mf::u32x4{qp[qi][s][p][0], qp[qi][s][p][1], qp[qi][s][p][2], qp[qi][s][p][3]});
+    };
+    // the six products, smallest first: planes (A, B)
+    constexpr int kProducts = 6;
+    constexpr int pa[kProducts] = {1, 2, 0, 1, 0, 0}, pb[kProducts] = {1, 0, 2, 0, 1, 0};
+
+#pragma unroll 1
+    for (uint32_t round = 0; round < rounds; ++round) {
+        const uint32_t c0 = start + (round * kPfGroups + grp) * kChunk;
+        group_sync(&arrived[grp], 8 * round + 4, lane);  // the previous chunk's reads are done
+        {
+            uint32_t bad_k = 0, bad_v = 0;
+            // K: dims 4 dq..+3 are half dq % 2 of lane group (dq % 8) / 2 in fragment (tile, dq / 8)
+            uint16_t *const kd = ks + (dq / 8) * 512 + (((dq % 8) / 2) * 16 + n) * 8 + (dq % 2) * 4;
 #pragma unroll
-        for (int k = 0; k < kPer; ++k) {
-            const uint32_t f = t + uint32_t(k) * kPfThreads, p = f / (kHead / 4), d4 = f % (kHead / 4);
-            const uint32_t at = min(c0 + p, hi);  // positions past the block's last re-read it
-            const size_t row = (size_t(at) * kKvHeads + kvh) * kHead;
-            *reinterpret_cast<float4 *>(ks + p * kRowStride + 4 * d4) = reinterpret_cast<const float4 *>(k_cache + row)[d4];
-            *reinterpret_cast<float4 *>(vs + p * kRowStride + 4 * d4) = reinterpret_cast<const float4 *>(v_cache + row)[d4];
+            for (int k = 0; k < 4; ++k) {
+                uint32_t w0[kPfPlanes], w1[kPfPlanes];
+                split3(kr[k].x, kr[k].y, w0);
+                split3(kr[k].z, kr[k].w, w1);
+                bad_k = pair_max(pair_max(bad_k, w0[0]), w1[0]);
+#pragma unroll
+                for (int p = 0; p < kPfPlanes; ++p) {
+                    *reinterpret_cast<u32x2 *>(kd + p * kPfPlane + k * 1024) = u32x2{w0[p], w1[p]};
+                }
+            }
+            // V: positions 4k..4k+3 of position tile `wave` are half wave % 2 of lane group k
+            // in fragment (dim tile, wave / 2)
+            uint16_t *const vd = vs + ((lane / 16) * 2 + wave / 2) * 512 + n * 8 + (wave % 2) * 4;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                uint32_t w0[kPfPlanes], w1[kPfPlanes];
+                split3(vr[4 * k], vr[4 * k + 1], w0);
+                split3(vr[4 * k + 2], vr[4 * k + 3], w1);
+                bad_v = pair_max(pair_max(bad_v, w0[0]), w1[0]);
+#pragma unroll
+                for (int p = 0; p < kPfPlanes; ++p) {
+                    *reinterpret_cast<u32x2 *>(vd + p * kPfPlane + k * 128) = u32x2{w0[p], w1[p]};
+                }
+            }
+            if (at_least<kPfKMax>(bad_k) || at_least<kPfVMax>(bad_v)) {
+                odd[grp][round % 2] = 1;
+            }
         }
-        __syncthreads();
+        group_sync(&arrived[grp], 8 * round + 8, lane);
+        if (round + 1 < rounds) {
+            request(round + 1);
+        }
+        const bool f32_chunk = (odd[grp][round % 2] | odd_query) != 0;
+        if (t == 0) {
+            odd[grp][(round + 1) % 2] = 0;  // set again only after the next two arrivals of this wave
+        }
+        if (f32_chunk) {
+            // (copies: the state itself stays in registers)
+            PfState s2 = st;
+            const PfQueries qs = {{qrow[0], qrow[1]}, {qfirst[0], qfirst[1]}, {qpos[0], qpos[1]}};
+            attn_chunk_f32(q, k_cache, v_cache, kvh, c0, hi, qs, n, g, s2);
+            st = s2;
+            // wait for the copies here: left to their first use, in the next chunk, the
+            // compiler waited there for the K and V requests ahead of it, on every path
+#pragma unroll
+            for (int qi = 0; qi < kPfTiles; ++qi) {
+                asm volatile("" : "+v"(st.m[qi]), "+v"(st.l[qi]), "+v"(st.o[qi][0]), "+v"(st.o[qi][1]),
+                             "+v"(st.o[qi][2]), "+v"(st.o[qi][3]));
+            }
+            continue;
+        }
 
         // S^T: [query tile][position tile], lane rows 4g..4g+3 = positions 16p + 4g + i
         f32x4 sc[kPfTiles][4];
 #pragma unroll
-        for (int p = 0; p < 4; ++p) {
+        for (int p2 = 0; p2 < 4; p2 += 2) {
 #pragma unroll
-            for (int qi = 0; qi < kPfTiles; ++qi) {
-                sc[qi][p] = f32x4{0.f, 0.f, 0.f, 0.f};
-            }
+            for (int s = 0; s < 2; ++s) {
+                bf16x8 a[2][kPfPlanes];
 #pragma unroll
-            for (int s4 = 0; s4 < 4; ++s4) {
-                const float4 a = *reinterpret_cast<const float4 *>(ks + (16 * p + n) * kRowStride + 16 * s4 + 4 * g);
+                for (int u = 0; u < 2; ++u) {
 #pragma unroll
-                for (int qi = 0; qi < kPfTiles; ++qi) {
-                    sc[qi][p] = mfma_f32(a.x, qv[qi][4 * s4], sc[qi][p]);
+                    for (int p = 0; p < kPfPlanes; ++p) {
+                        a[u][p] = frag(ks, p, 2 * (p2 + u) + s);
+                    }
                 }
 #pragma unroll
-                for (int qi = 0; qi < kPfTiles; ++qi) {
-                    sc[qi][p] = mfma_f32(a.y, qv[qi][4 * s4 + 1], sc[qi][p]);
-                }
+                for (int x = 0; x < kProducts; ++x) {
 #pragma unroll
-                for (int qi = 0; qi < kPfTiles; ++qi) {
-                    sc[qi][p] = mfma_f32(a.z, qv[qi][4 * s4 + 2], sc[qi][p]);
-                }
+                    for (int u = 0; u < 2; ++u) {
 #pragma unroll
-                for (int qi = 0; qi < kPfTiles; ++qi) {
-                    sc[qi][p] = mfma_f32(a.w, qv[qi][4 * s4 + 3], sc[qi][p]);
+                        for (int qi = 0; qi < kPfTiles; ++qi) {
+                            sc[qi][p2 + u] = mf::mfma(a[u][pa[x]], q_frag(qi, s, pb[x]),
+                                                      s == 0 && x == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : sc[qi][p2 + u]);
+                        }
+                    }
                 }
             }
         }
-        // scores (1/sqrt(64) = 0.125, exact), mask, online softmax; sc becomes P^T
+        // mask, online softmax; sc becomes P^T
+        const bool whole = c0 + kChunk - 1 <= first + block0 && c0 >= span_of(hi, layer_index).first;
 #pragma unroll
         for (int qi = 0; qi < kPfTiles; ++qi) {
-            float cmax = -INFINITY;
+            if (!whole) {  // (uniform) some position is outside some query's span
+#pragma unroll
+                for (int p = 0; p < 4; ++p) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const uint32_t at = c0 + 16 * p + 4 * g + i;
+                        sc[qi][p][i] = at >= qfirst[qi] && at <= qpos[qi] ? sc[qi][p][i] : kPfMasked;
+                    }
+                }
+            }
+            float cmax = sc[qi][0][0];
 #pragma unroll
             for (int p = 0; p < 4; ++p) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const uint32_t at = c0 + 16 * p + 4 * g + i;
-                    const bool in = at >= qfirst[qi] && at <= qpos[qi];
-                    const float s = in ? sc[qi][p][i] * 0.125f : -INFINITY;
-                    sc[qi][p][i] = s;
-                    cmax = fmaxf(cmax, s);
+                    cmax = fmaxf(cmax, sc[qi][p][i]);
                 }
             }
-            cmax = fmaxf(cmax, __shfl_xor(cmax, 16));
-            cmax = fmaxf(cmax, __shfl_xor(cmax, 32));
-            const float m2 = fmaxf(m[qi], cmax);
-            const float scale = expf(m[qi] - m2);
+            const float m2 = pf_rescale(st, qi, cmax);
             float lsum = 0.0f;
 #pragma unroll
             for (int p = 0; p < 4; ++p) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const float s = sc[qi][p][i];
-                    const float x = s == -INFINITY ? 0.0f : expf(s - m2);
+                    const float x = __builtin_amdgcn_exp2f(sc[qi][p][i] - m2);
                     sc[qi][p][i] = x;
                     lsum += x;
                 }
             }
-            l[qi] = l[qi] * scale + lsum;
-            m[qi] = m2;
-#pragma unroll
-            for (int mt = 0; mt < 4; ++mt) {
-                o[qi][mt] *= scale;
-            }
+            st.l[qi] += lsum;
         }
         // O^T += V^T P^T
 #pragma unroll
-        for (int mt = 0; mt < 4; ++mt) {
+        for (int h = 0; h < 2; ++h) {
+            mf::u32x4 pp[kPfTiles][kPfPlanes];
 #pragma unroll
-            for (int p = 0; p < 4; ++p) {
+            for (int qi = 0; qi < kPfTiles; ++qi) {
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const float a = vs[(16 * p + 4 * g + j) * kRowStride + 16 * mt + n];
+                for (int e = 0; e < 4; ++e) {
+                    uint32_t w[kPfPlanes];
+                    split3(sc[qi][2 * h + e / 2][2 * (e % 2)], sc[qi][2 * h + e / 2][2 * (e % 2) + 1], w);
 #pragma unroll
-                    for (int qi = 0; qi < kPfTiles; ++qi) {
-                        o[qi][mt] = mfma_f32(a, sc[qi][p][j], o[qi][mt]);
+                    for (int p = 0; p < kPfPlanes; ++p) {
+                        pp[qi][p][e] = w[p];
+                    }
+                }
+            }
+#pragma unroll
+            for (int m2 = 0; m2 < 4; m2 += 2) {
+                bf16x8 a[2][kPfPlanes];
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+#pragma unroll
+                    for (int p = 0; p < kPfPlanes; ++p) {
+                        a[u][p] = frag(vs, p, 2 * (m2 + u) + h);
+                    }
+                }
+#pragma unroll
+                for (int x = 0; x < kProducts; ++x) {
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+#pragma unroll
+                        for (int qi = 0; qi < kPfTiles; ++qi) {
+                            st.o[qi][m2 + u] = mf::mfma(a[u][pa[x]], mf::as_bf16x8v(pp[qi][pb[x]]), st.o[qi][m2 + u]);
+                        }
                     }
                 }
             }
         }
     }
+
+    // group 1 hands its state to group 0's wave of the same queries through LDS
+    constexpr int kState = 18;  // per lane and query tile: m, l and 16 of O
+    float *const hand = reinterpret_cast<float *>(&kv[0][0][0][0]) + size_t(wave) * kPfTiles * kState * 64 + lane;
+    static_assert(sizeof(float) * 4 * kPfTiles * kState * 64 <= sizeof(kv), "the handed state fits the staged planes");
+    __syncthreads();
+    if (grp == 1) {
 #pragma unroll
-    for (int qi = 0; qi < kPfTiles; ++qi) {
-        float den = l[qi] + __shfl_xor(l[qi], 16);
-        den = den + __shfl_xor(den, 32);
-        if (qlocal[qi] < tokens) {
-            float *dst = out + (size_t(qlocal[qi]) * kQHeads + qhead[qi]) * kHead;
+        for (int qi = 0; qi < kPfTiles; ++qi) {
+            float *d = hand + qi * kState * 64;
+            d[0] = st.m[qi];
+            d[64] = st.l[qi];
 #pragma unroll
             for (int mt = 0; mt < 4; ++mt) {
-                const f32x4 v = o[qi][mt];
-                *reinterpret_cast<float4 *>(dst + 16 * mt + 4 * g) =
-                    make_float4(v[0] / den, v[1] / den, v[2] / den, v[3] / den);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    d[(2 + 4 * mt + i) * 64] = st.o[qi][mt][i];
+                }
+            }
+        }
+    }
+    __syncthreads();
+    if (grp == 1) {
+        return;
+    }
+#pragma unroll
+    for (int qi = 0; qi < kPfTiles; ++qi) {
+        const float *d = hand + qi * kState * 64;
+        const float m1 = d[0];
+        const float m = fmaxf(st.m[qi], m1);
+        const float w0 = __builtin_amdgcn_exp2f(st.m[qi] - m), w1 = __builtin_amdgcn_exp2f(m1 - m);
+        float den = st.l[qi] * w0 + d[64] * w1;
+        den += __shfl_xor(den, 16);
+        den += __shfl_xor(den, 32);
+        if (live[qi]) {
+            float *dst = out + size_t(qrow[qi]) * kHead;
+#pragma unroll
+            for (int mt = 0; mt < 4; ++mt) {
+                float v[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    v[i] = (st.o[qi][mt][i] * w0 + d[(2 + 4 * mt + i) * 64] * w1) / den;
+                }
+                *reinterpret_cast<float4 *>(dst + 16 * mt + 4 * g) = make_float4(v[0], v[1], v[2], v[3]);
             }
         }
     }
