@@ -72,6 +72,31 @@ def test_q8_matmul_residual_and_no_bias(dev):
     t.free()
 
 
+# One call per tile shape and K split that the launch picks (on 256 CUs: 1x1, 1x2, 2x2,
+# 2x3, 2x5 on 8 waves; 2x5 on 4; 4x3 and 4x5 on 8 and on 4 waves), with a last row group and
+# a last token group that are partly empty.  Against 64 bits: the planes hold 2^-22 of each
+# value and a row sums at most 4096 products, so 1e-6 relative covers both.
+@pytest.mark.parametrize("rows,cols,tokens", [
+    (2880, 4096, 15), (5104, 2880, 16), (5104, 2880, 31), (2864, 4096, 125), (5104, 2880, 125), (5104, 2880, 289),
+    (2864, 4096, 250), (5104, 2880, 250), (2864, 4096, 509), (5104, 2880, 509), (5104, 2880, 1)])
+def test_q8_matmul_tile_shapes(dev, rows, cols, tokens):
+    blocks = O.synth_q8_0(31, cols + tokens, rows * cols // 32)
+    x = O.synth_normal(32, cols + tokens, tokens * cols).reshape(tokens, cols)
+    bias, resid = O.synth_normal(33, cols, rows), O.synth_normal(34, tokens, tokens * rows).reshape(tokens, rows)
+    t = dev.q8_upload(blocks, rows, cols)
+    xb, bb, rb = dev.upload(x), dev.upload(bias), dev.upload(resid)
+    ob = dev.upload(np.full((tokens + 1) * rows, 7.0, np.float32))
+    dev.matmul_q8_0(t, bb, xb, tokens, rb, ob)
+    got = ob.download(np.float32).reshape(tokens + 1, rows)
+    assert np.all(got[tokens] == 7.0)  # nothing past the last token
+    exact = x.astype(np.float64) @ q8_dense(blocks, rows, cols).T + bias + resid
+    for p in range(tokens):
+        assert O.rel_l2(got[p], exact[p]) < 1e-6, p
+    for b in (xb, bb, rb, ob):
+        b.free()
+    t.free()
+
+
 def test_q8_matmul_rejects_small_workspace(dev):
     import ctypes as C
     import ttlab_amd

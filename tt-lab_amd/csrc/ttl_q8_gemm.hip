@@ -7,8 +7,7 @@
 // rows 4g..4g+3 of column l%16):
 //  - one K step is one Q8_0 block of 32 columns; lane group g holds offsets 8g..8g+7;
 //  - A is 16 tokens: token t's f32 activations times 2^k_t as two f16 planes
-//    (mf::split_f16x2, k_t = mf::row_shift of the row's largest finite |x|), staged
-//    through LDS;
+//    (mf::split_f16x2, k_t = mf::row_shift of the row's largest finite |x|);
 //  - B is 16 weight rows: the int8 codes, exact in f16 (|q| <= 128 < 2^11);
 //  - D[token][row]: a lane holds four tokens of one row, so the block's fp16 scale is
 //    one value per lane, applied after the block: acc += d * (A0 B + A1 B).
@@ -19,10 +18,18 @@
 // the products sequentially from the bias (d q rounds to nothing: it has at most 19
 // significant bits), so results agree to f32 rounding, not bit for bit.
 //
-// Workspace: token fragments [token tile of 64][plane][step][16-token sub-tile][lane][16 B]
-// (steps past the last block -- K = 2880 has 90 blocks, padded to 92 -- hold zero tokens,
-// and their row scales are zero), then the tokens' shifts k_t [tiles x 64] (int32), unless
-// the caller passes them (ttl_matmul_q8_0_shifted).
+// What bounds it: the projections are small (15 GFLOP at 512 tokens, 24 us of the card's
+// library GEMM rate with both planes), so the split matters more than the inner loop.  One
+// workgroup used to take all of K for 64 tokens x 4 row tiles: at 77 tokens 90 workgroups
+// each ran a chain of 128 steps (46 us), and at 512 every wave read all token fragments
+// from LDS for one row tile.  K now goes over the waves of a workgroup and the tile shape
+// follows the call's size (launch_gemm_for).  Whole calls, 5120 x 2880 at 512 tokens: 62.5
+// to 45.2 us; 2880 x 4096 at 512 tokens 83 to 49 us, at 77 tokens 51 to 22 us.
+//
+// Workspace: token fragments [16-token sub-tile][step][plane][lane][16 B] (steps past the
+// last block -- K = 2880 has 90 blocks, padded to 92 -- hold zero tokens, and their row
+// scales are zero), then the tokens' shifts k_t (int32), unless the caller passes them
+// (ttl_matmul_q8_0_shifted).
 #include "ttl_mfma.hpp"
 
 #include <hip/hip_fp16.h>
@@ -33,64 +40,83 @@ using mf::f16x8;
 using mf::f32x4;
 
 constexpr int kPlanes = 2;
-constexpr int kSub = 4;  // 16-token sub-tiles per 64-token tile
-constexpr int kTileTokens = 16 * kSub;
-constexpr int kStageSteps = 2;  // K steps per LDS stage
-constexpr int kWaves = 4;
-// 16-row weight tiles per wave: one.  The projections have 2880 and 5120 rows, so more
-// tiles per workgroup leave CUs idle at a 512-token prompt (measured: one tile per wave
-// beat two and three in the layer-major prefill).
-constexpr int kRowTiles = 1;
-constexpr int kLook = 4;  // token fragments read from LDS this many ahead
+constexpr int kSubTokens = 16;  // tokens of one fragment
 
 template <int K>
 struct Shape {
     static constexpr int blocks = K / 32;
     static constexpr int quads = (blocks + 3) / 4;
     static constexpr int steps = quads * 4;
-    static constexpr int stages = steps / kStageSteps;
-    static constexpr size_t plane_bytes = size_t(steps) * kSub * mf::frag_bytes;
-    static constexpr size_t tile_bytes = kPlanes * plane_bytes;
-    static constexpr int stage_frags = kPlanes * kStageSteps * kSub;
-    static constexpr int stage_chunks = stage_frags * 64;  // 16-byte pieces
+    // one 16-token sub-tile: [step][plane] fragments
+    static constexpr size_t sub_bytes = size_t(steps) * kPlanes * mf::frag_bytes;
 };
 
-// Token fragments of one (step, tile): thread (sub-tile m, lane (t, g)) converts
-// x[64 tile + 16 m + t][32 step + 8 g .. + 7] times 2^shift[token] (zero past the tokens
-// or the row end).
-template <int K>
-__global__ __launch_bounds__(kSub * 64) void q8_gather_kernel(const float *__restrict__ x, uint32_t tokens,
-                                                              const int32_t *__restrict__ shift,
-                                                              uint8_t *__restrict__ frags) {
+// Token fragments, one wave per token: lane l requests the row's pieces of 8 values l, l + 64,
+// ... at once, takes the largest finite |x| over the wave unless the shifts are given, and
+// writes piece j = 4 step + g times 2^shift as two planes (16 bytes each, lane (t, g) of its
+// sub-tile's fragment; the four tokens of a workgroup are neighbours there).  Tokens past
+// the count and steps past the row are zero.  Replaces a launch for the shifts and one with
+// a thread per piece: 4.6 + 5.2 us at 512 x 4096, one launch of 5.0 us.
+constexpr int kGatherWaves = 4;
+template <int K, bool SHIFTED>
+__global__ __launch_bounds__(kGatherWaves * 64) void q8_gather_kernel(const float *__restrict__ x, uint32_t tokens,
+                                                                      int32_t *__restrict__ shift,
+                                                                      uint8_t *__restrict__ frags) {
     using S = Shape<K>;
-    const uint32_t step = blockIdx.x, tile = blockIdx.y;
-    const uint32_t m = threadIdx.x / 64, lane = threadIdx.x % 64, g = lane / 16;
-    const uint32_t token = tile * kTileTokens + m * 16 + lane % 16;
-    const int k = shift[token < tokens ? token : 0];
-    float v[8];
-    if (token < tokens && step < uint32_t(S::blocks)) {
-        const float4 *p = reinterpret_cast<const float4 *>(x + size_t(token) * K + step * 32 + 8 * g);
-        const float4 lo = p[0], hi = p[1];
-        v[0] = lo.x;
-        v[1] = lo.y;
-        v[2] = lo.z;
-        v[3] = lo.w;
-        v[4] = hi.x;
-        v[5] = hi.y;
-        v[6] = hi.z;
-        v[7] = hi.w;
-    } else {
+    constexpr int pieces = K / 8, per = (S::steps * 4 + 63) / 64;
+    const uint32_t token = blockIdx.x * kGatherWaves + threadIdx.x / 64, lane = threadIdx.x % 64;
+    const bool live = token < tokens;
+    const float4 *row = reinterpret_cast<const float4 *>(x + size_t(live ? token : 0) * K);
+    float v[per][8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            v[j] = 0.0f;
+    for (int i = 0; i < per; ++i) {
+        const uint32_t j = min(lane + 64u * i, uint32_t(pieces - 1));
+        const float4 lo = row[2 * j], hi = row[2 * j + 1];
+        v[i][0] = lo.x;
+        v[i][1] = lo.y;
+        v[i][2] = lo.z;
+        v[i][3] = lo.w;
+        v[i][4] = hi.x;
+        v[i][5] = hi.y;
+        v[i][6] = hi.z;
+        v[i][7] = hi.w;
+    }
+    int k;
+    if constexpr (SHIFTED) {
+        k = shift[live ? token : 0];
+    } else {
+        float m = 0.0f;
+#pragma unroll
+        for (int i = 0; i < per; ++i) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                m = mf::finite_max(m, v[i][e]);
+            }
+        }
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) {
+            m = __builtin_fmaxf(m, __shfl_xor(m, d));
+        }
+        k = mf::row_shift(m);
+        if (live && lane == 0) {
+            shift[token] = k;
         }
     }
-    uint4 out[kPlanes];
-    mf::split_f16x2(v, k, out);
-    uint8_t *dst = frags + size_t(tile) * S::tile_bytes + (size_t(step) * kSub + m) * mf::frag_bytes + lane * 16;
+    uint8_t *dst = frags + size_t(token / kSubTokens) * S::sub_bytes + (token % kSubTokens) * 16;
 #pragma unroll
-    for (int p = 0; p < kPlanes; ++p) {
-        *reinterpret_cast<uint4 *>(dst + size_t(p) * S::plane_bytes) = out[p];
+    for (int i = 0; i < per; ++i) {
+        const uint32_t j = lane + 64u * i;
+        if (j >= uint32_t(S::steps * 4)) {
+            continue;
+        }
+        uint4 out[kPlanes] = {make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0)};
+        if (live && j < uint32_t(pieces)) {
+            mf::split_f16x2(v[i], k, out);
+        }
+#pragma unroll
+        for (int p = 0; p < kPlanes; ++p) {
+            *reinterpret_cast<uint4 *>(dst + (size_t(j / 4) * kPlanes + p) * mf::frag_bytes + (j % 4) * 256) = out[p];
+        }
     }
 }
 
@@ -104,8 +130,8 @@ __device__ inline f16x8 int8_f16(uint2 c) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         const uint32_t w = (k < 2 ? c.x : c.y) ^ 0x80808080u;
-        const uint32_t b = k % 2 == 0 ? w : w >> 16;  // the two codes in bytes 0 and 1
-        const uint32_t h = (b & 0xffu) | ((b & 0xff00u) << 8) | 0x64006400u;
+        // bytes (0x64, code 2k + 1, 0x64, code 2k): one byte permutation of (w, 0x64...)
+        const uint32_t h = __builtin_amdgcn_perm(0x64646464u, w, k % 2 == 0 ? 0x04010400u : 0x04030402u);
         const f16x2v v = __builtin_bit_cast(f16x2v, h) - bias;
         r[2 * k] = v[0];
         r[2 * k + 1] = v[1];
@@ -124,225 +150,262 @@ struct GemmArgs {
     uint32_t rows, row_tiles, tokens;
 };
 
-// One workgroup: a 64-token tile x 4 * kRowTiles weight-row tiles; wave w takes row
-// tiles (group * 4 + w) * kRowTiles + j.  Token fragments go through LDS in stages of two K
-// steps (double-buffered); each wave's weight codes and scales are requested one
-// quad (4 steps) ahead.
-template <int K>
-__global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(2))) void q8_gemm_kernel(GemmArgs a) {
+// One workgroup: SUBS 16-token sub-tiles x TILES 16-row weight tiles, its KW waves each a
+// range of the K quads over the whole of that (every fragment and code is requested once per
+// workgroup, straight into registers: no LDS copy and no barrier in the loop), one step
+// ahead.  The waves' sums are added in LDS in wave order, MS sub-tiles at a time.
+template <int K, int SUBS, int TILES, int KW>
+__global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(2))) void q8_gemm_kernel(GemmArgs a) {
     using S = Shape<K>;
-    constexpr int kThreads = kWaves * 64;
-    constexpr int kPer = S::stage_chunks / kThreads;
-    static_assert(S::stage_chunks % kThreads == 0, "the stager moves whole pieces");
-    __shared__ mf::u32x4 lds[2][S::stage_chunks];
-    const uint32_t t = threadIdx.x, wave = t / 64, lane = t % 64, n = lane % 16, g = lane / 16;
-    const uint32_t tile = blockIdx.y;
-    const uint8_t *frags = a.frags + size_t(tile) * S::tile_bytes;
+    constexpr int per = (S::quads + KW - 1) / KW;  // quads per wave
+    constexpr int MS = SUBS < 2 || KW > 4 ? 1 : 2;
+    constexpr int kRows = TILES * 16, kStride = kRows + 4;  // + 4: the lane groups' rows in other banks
+    __shared__ float part[KW][MS * kSubTokens * kStride];
+    // (the wave as a scalar: every address is a uniform base plus the lane's constant offset)
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const uint32_t lane = threadIdx.x % 64, n = lane % 16, g = lane / 16;
+    const uint32_t sub0 = blockIdx.y * SUBS, subs = (a.tokens + kSubTokens - 1) / kSubTokens;
+    const uint32_t q0 = wave * per, q1 = min(q0 + per, uint32_t(S::quads));
 
-    // this wave's weight row tiles (tiles past the matrix re-read tile 0; not written)
-    const uint8_t *cp[kRowTiles];
-    const uint16_t *sp[kRowTiles];
-    bool ok[kRowTiles];
-    uint32_t row[kRowTiles];
+    // sub-tiles past the tokens and row tiles past the matrix re-read the last (not written)
+    const uint8_t *fp[SUBS];
 #pragma unroll
-    for (int j = 0; j < kRowTiles; ++j) {
-        const uint32_t rt = (blockIdx.x * kWaves + wave) * kRowTiles + j;
-        ok[j] = rt < a.row_tiles;
-        const uint32_t rts = ok[j] ? rt : 0;
-        row[j] = rts * 16 + n;
-        // bytes 8g..8g+7 of row n's block: half g / 2 (q8::code_offset), 8 (g % 2) into it
-        cp[j] = a.codes + size_t(rts) * S::blocks * 512 + (g / 2) * 256 + n * 16 + 8 * (g % 2);
-        sp[j] = a.row_scales + size_t(row[j]) * S::steps;
+    for (int m = 0; m < SUBS; ++m) {
+        fp[m] = a.frags + size_t(min(sub0 + m, subs - 1)) * S::sub_bytes;
     }
-
-    // stage j: K steps 2j, 2j+1 of all planes and sub-tiles, LDS order [plane][step][sub][lane]
-    mf::u32x4 st[kPer];
-    auto stage_load = [&](int j) __attribute__((always_inline)) {
+    uint32_t rt[TILES];
 #pragma unroll
-        for (int k = 0; k < kPer; ++k) {
-            const uint32_t c = t + uint32_t(k) * kThreads;
-            const uint32_t p = c / (kStageSteps * kSub * 64), within = c % (kStageSteps * kSub * 64);
-            st[k] = *reinterpret_cast<const mf::u32x4 *>(frags + size_t(p) * S::plane_bytes +
-                                                       size_t(j) * kStageSteps * kSub * mf::frag_bytes +
-                                                       size_t(within) * 16);
+    for (int t = 0; t < TILES; ++t) {
+        rt[t] = min(uint32_t(blockIdx.x * TILES + t), a.row_tiles - 1);
+    }
+    // bytes 8g..8g+7 of row n's block: half g / 2 (q8::code_offset), 8 (g % 2) into it
+    const uint32_t code_at = (g / 2) * 32 + n * 2 + g % 2, scale_at = n * (S::steps / 4);  // in uint2
+
+    f16x8 xf[2][SUBS][kPlanes];
+    uint2 qc[2][TILES], qs[2][TILES];
+    auto load_step = [&](uint32_t s, f16x8(&x)[SUBS][kPlanes], uint2(&c)[TILES]) __attribute__((always_inline)) {
+        const uint32_t b = min(s, uint32_t(S::blocks - 1));
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+            c[t] = reinterpret_cast<const uint2 *>(a.codes + (size_t(rt[t]) * S::blocks + b) * 512)[code_at];
+        }
+#pragma unroll
+        for (int m = 0; m < SUBS; ++m) {
+#pragma unroll
+            for (int p = 0; p < kPlanes; ++p) {
+                x[m][p] = reinterpret_cast<const f16x8 *>(fp[m] + (size_t(s) * kPlanes + p) * mf::frag_bytes)[lane];
+            }
         }
     };
-    auto stage_store = [&](mf::u32x4 *dst) __attribute__((always_inline)) {
+    auto load_scales = [&](uint32_t q, uint2(&d)[TILES]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int k = 0; k < kPer; ++k) {
-            dst[t + uint32_t(k) * kThreads] = st[k];
+        for (int t = 0; t < TILES; ++t) {
+            d[t] = reinterpret_cast<const uint2 *>(a.row_scales + size_t(rt[t]) * 16 * S::steps + 4 * q)[scale_at];
         }
     };
 
-    // weight codes and scales of one quad: [row tile][step], [row tile] (4 fp16)
-    uint2 qc[2][kRowTiles][4];
-    uint2 qs[2][kRowTiles];
-    auto load_quad = [&](int q, uint2(&c)[kRowTiles][4], uint2(&s)[kRowTiles]) __attribute__((always_inline)) {
+    f32x4 acc[SUBS][TILES];
 #pragma unroll
-        for (int j = 0; j < kRowTiles; ++j) {
+    for (int m = 0; m < SUBS; ++m) {
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+            acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+    // One region per weight tile: the block's MFMAs of all sub-tiles, and between them, in
+    // the 12 cycles that each leaves the VALU, the scaling of the tile before and the
+    // decoding of the tile after (w, d: of the tile to multiply; pend, pend_d: products to scale).
+    f16x8 w;
+    float d = 0.0f, pend_d = 0.0f;
+    f32x4 pend[SUBS];
+#pragma unroll
+    for (int m = 0; m < SUBS; ++m) {
+        pend[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    auto scale_of = [&](int k, const uint2 &four) __attribute__((always_inline)) {
+        return __half2float(__ushort_as_half(uint16_t((k < 2 ? four.x : four.y) >> (16 * (k % 2)))));
+    };
+    // step k of its quad; kn, cn, sn: the next step's place in its quad, first codes and scales
+    auto step = [&](int k, const f16x8(&x)[SUBS][kPlanes], const uint2(&c)[TILES], const uint2(&s)[TILES], int kn,
+                    const uint2 &cn, const uint2 &sn) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+            f32x4 cur[SUBS];
+#pragma unroll
+            for (int m = 0; m < SUBS; ++m) {
+                cur[m] = mf::mfma(x[m][0], w, f32x4{0.f, 0.f, 0.f, 0.f});
+            }
+#pragma unroll
+            for (int m = 0; m < SUBS; ++m) {
+                cur[m] = mf::mfma(x[m][1], w, cur[m]);
+            }
+            constexpr int last = TILES - 1;
+#pragma unroll
+            for (int m = 0; m < SUBS; ++m) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    acc[m][t == 0 ? last : t - 1][e] = fmaf(pend_d, pend[m][e], acc[m][t == 0 ? last : t - 1][e]);
+                }
+            }
+            const f16x8 wn = int8_f16(t < last ? c[t < last ? t + 1 : 0] : cn);
+            const float dn = t < last ? scale_of(k, s[t < last ? t + 1 : 0]) : scale_of(kn, sn);
+#pragma unroll
+            for (int i = 0; i < SUBS * kPlanes; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA,
+                __builtin_amdgcn_sched_group_barrier(0x002, SUBS == 4 ? 4 : (SUBS == 2 ? 6 : 9), 0);  // then VALU
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int m = 0; m < SUBS; ++m) {
+                // an empty statement that takes the sum in registers here: the compiler
+                // otherwise sinks these updates and keeps every block product live
+                asm volatile("" : "+v"(acc[m][t == 0 ? last : t - 1]));
+                pend[m] = cur[m];
+            }
+            pend_d = d;
+            w = wn;
+            d = dn;
+        }
+    };
+
+    if (q0 < q1) {
+        load_scales(q0, qs[0]);
+        load_step(4 * q0, xf[0], qc[0]);
+        w = int8_f16(qc[0][0]);
+        d = scale_of(0, qs[0][0]);
+        // (requests past the range repeat its last quad or step)
+        auto quad = [&](uint32_t q, const uint2(&s)[TILES], uint2(&next)[TILES]) __attribute__((always_inline)) {
+            load_scales(min(q + 1, q1 - 1), next);
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                const uint32_t b = min(uint32_t(4 * q + k), uint32_t(S::blocks - 1));
-                c[j][k] = *reinterpret_cast<const uint2 *>(cp[j] + size_t(b) * 512);
-            }
-            s[j] = *reinterpret_cast<const uint2 *>(sp[j] + 4 * q);
-        }
-    };
-
-    // acc: the scaled sum so far.  The MFMAs of a K step go to cur; the scale FMAs of
-    // a step run one step later, from pend (the previous step's sums) and pend_d, so the
-    // VALU never waits on an MFMA result that was just issued.
-    f32x4 acc[kSub][kRowTiles], cur[kSub][kRowTiles], pend[kSub][kRowTiles];
-    float dcur[kRowTiles], pend_d[kRowTiles];
-#pragma unroll
-    for (int j = 0; j < kRowTiles; ++j) {
-        dcur[j] = 0.0f;
-        pend_d[j] = 0.0f;
-#pragma unroll
-        for (int m = 0; m < kSub; ++m) {
-            acc[m][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-            pend[m][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
-    }
-
-    stage_load(0);
-    load_quad(0, qc[0], qs[0]);
-    stage_store(lds[0]);
-    __syncthreads();
-    stage_load(1);
-
-    // the MFMAs of quad q (stages 2q, 2q+1) with its codes c and scales s
-    auto compute_quad = [&](int q, const uint2(&c)[kRowTiles][4], const uint2(&s)[kRowTiles])
-                            __attribute__((always_inline)) {
-#pragma unroll
-        for (int h = 0; h < 4 / kStageSteps; ++h) {
-            const int stage = 2 * q + h;
-            const mf::u32x4 *buf = lds[stage % 2];
-            constexpr int SF = S::stage_frags;
-            // fragment order within a stage: step, plane, sub-tile (the four sub-tiles'
-            // MFMAs are independent, so consecutive MFMAs never wait on each other)
-            auto frag = [&](int f) __attribute__((always_inline)) {
-                const int ls = f / (kSub * kPlanes), p = (f / kSub) % kPlanes, m = f % kSub;
-                return __builtin_bit_cast(f16x8, buf[((p * kStageSteps + ls) * kSub + m) * 64 + lane]);
-            };
-            f16x8 ring[kLook];
-#pragma unroll
-            for (int d = 0; d < kLook; ++d) {
-                ring[d] = frag(d);
-            }
-            f16x8 w[kRowTiles];
-#pragma unroll
-            for (int f = 0; f < SF; ++f) {
-                const f16x8 av = ring[f % kLook];
-                if (f + kLook < SF) {
-                    ring[f % kLook] = frag(f + kLook);
-                }
-                const int ls = f / (kSub * kPlanes), p = (f / kSub) % kPlanes, m = f % kSub;
-                const int k = h * kStageSteps + ls;  // step within the quad
-                if (f % (kSub * kPlanes) == 0) {
-#pragma unroll
-                    for (int j = 0; j < kRowTiles; ++j) {
-                        w[j] = int8_f16(c[j][k]);
-                        const uint32_t word = k < 2 ? s[j].x : s[j].y;
-                        pend_d[j] = dcur[j];
-                        dcur[j] = __half2float(__ushort_as_half(uint16_t(word >> (16 * (k % 2)))));
-                    }
-                }
-#pragma unroll
-                for (int j = 0; j < kRowTiles; ++j) {
-                    cur[m][j] = mf::mfma(av, w[j], p == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : cur[m][j]);
-                    if (p == kPlanes - 1) {
-                        // the previous step's block sum, scaled by its fp16 d
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            acc[m][j][e] = fmaf(pend_d[j], pend[m][j][e], acc[m][j][e]);
-                        }
-                        // an empty statement that takes the sum in registers here: the
-                        // compiler otherwise sinks these updates below the stage's MFMAs
-                        // and keeps every block product live
-                        asm volatile("" : "+v"(acc[m][j]));
-                        pend[m][j] = cur[m][j];
-                    }
-                }
-                // keep the ring's order: without this the scheduler hoists every LDS
-                // read of the stage and runs out of registers
+                load_step(min(4 * q + k + 1, 4 * q1 - 1), xf[(k + 1) % 2], qc[(k + 1) % 2]);
                 __builtin_amdgcn_sched_barrier(0);
+                step(k, xf[k % 2], qc[k % 2], s, (k + 1) % 4, qc[(k + 1) % 2][0], k < 3 ? s[0] : next[0]);
             }
-            // end of stage: publish the next, fetch the one after
-            if (stage + 1 < S::stages) {
-                stage_store(lds[(stage + 1) % 2]);
-            }
-            __syncthreads();
-            if (stage + 2 < S::stages) {
-                stage_load(stage + 2);
-            }
-        }
-    };
-
+        };
 #pragma unroll 1
-    for (int q = 0; q < S::quads; q += 2) {
-        load_quad(min(q + 1, S::quads - 1), qc[1], qs[1]);
-        compute_quad(q, qc[0], qs[0]);
-        if (q + 1 < S::quads) {
-            load_quad(min(q + 2, S::quads - 1), qc[0], qs[0]);
-            compute_quad(q + 1, qc[1], qs[1]);
+        for (uint32_t q = q0; q < q1; q += 2) {
+            quad(q, qs[0], qs[1]);
+            if (q + 1 < q1) {
+                quad(q + 1, qs[1], qs[0]);
+            }
         }
-    }
-    // the last step's sums
+        // the last tile of the last step
 #pragma unroll
-    for (int j = 0; j < kRowTiles; ++j) {
-#pragma unroll
-        for (int m = 0; m < kSub; ++m) {
+        for (int m = 0; m < SUBS; ++m) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                acc[m][j][e] = fmaf(dcur[j], pend[m][j][e], acc[m][j][e]);
+                acc[m][TILES - 1][e] = fmaf(pend_d, pend[m][e], acc[m][TILES - 1][e]);
             }
         }
     }
 
-    // D rows 4g..4g+3 of sub-tile m are tokens; the lane's column is row[j]
-    int ks[kSub][4];  // the shifts of the lane's 16 tokens (tokens past the count read token 0's)
+    // D rows 4g..4g+3 of sub-tile m are tokens; the lane's column is weight row n
 #pragma unroll
-    for (int m = 0; m < kSub; ++m) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const uint32_t token = tile * kTileTokens + m * 16 + 4 * g + e;
-            ks[m][e] = a.shift[token < a.tokens ? token : 0u];
+    for (int m0 = 0; m0 < SUBS; m0 += MS) {
+        if (m0 > 0) {
+            __syncthreads();
         }
-    }
 #pragma unroll
-    for (int j = 0; j < kRowTiles; ++j) {
-        if (!ok[j]) {
-            continue;
-        }
-        const float bv = a.bias ? a.bias[row[j]] : 0.0f;
+        for (int m = 0; m < MS; ++m) {
 #pragma unroll
-        for (int m = 0; m < kSub; ++m) {
+            for (int t = 0; t < TILES; ++t) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const uint32_t token = tile * kTileTokens + m * 16 + 4 * g + e;
-                if (token < a.tokens) {
-                    const size_t o = size_t(token) * a.rows + row[j];
-                    const float sum = __builtin_amdgcn_ldexpf(acc[m][j][e], -ks[m][e]);
-                    float v = a.bias ? bv + sum : sum;
-                    if (a.residual) {
-                        v = a.residual[o] + v;
-                    }
-                    a.out[o] = v;
+                for (int e = 0; e < 4; ++e) {
+                    part[wave][(m * kSubTokens + 4 * g + e) * kStride + t * 16 + n] = acc[m0 + m][t][e];
                 }
+            }
+        }
+        __syncthreads();
+        for (uint32_t i = threadIdx.x; i < uint32_t(MS * kSubTokens * kRows); i += KW * 64) {
+            const uint32_t lt = i / kRows, lr = i % kRows;
+            const uint32_t token = (sub0 + m0) * kSubTokens + lt, row = blockIdx.x * kRows + lr;
+            if (token < a.tokens && row < a.rows) {
+                float sum = part[0][lt * kStride + lr];
+#pragma unroll
+                for (int w = 1; w < KW; ++w) {
+                    sum += part[w][lt * kStride + lr];
+                }
+                const size_t o = size_t(token) * a.rows + row;
+                float v = __builtin_amdgcn_ldexpf(sum, -a.shift[token]);
+                if (a.bias) {
+                    v = a.bias[row] + v;
+                }
+                if (a.residual) {
+                    v = a.residual[o] + v;
+                }
+                a.out[o] = v;
             }
         }
     }
 }
 
+// (room for whole groups of four sub-tiles)
+constexpr uint32_t kRoomTokens = 4 * kSubTokens;
 template <int K>
 size_t frag_bytes_for(uint32_t tokens) {
-    return (size_t((tokens + kTileTokens - 1) / kTileTokens) * Shape<K>::tile_bytes + 255) & ~size_t(255);
+    return (size_t((tokens + kRoomTokens - 1) / kRoomTokens) * 4 * Shape<K>::sub_bytes + 255) & ~size_t(255);
 }
 
 template <int K>
 size_t workspace_for(uint32_t tokens) {
-    return frag_bytes_for<K>(tokens) + size_t((tokens + kTileTokens - 1) / kTileTokens) * kTileTokens * 4;
+    return frag_bytes_for<K>(tokens) + size_t((tokens + kRoomTokens - 1) / kRoomTokens) * kRoomTokens * 4;
+}
+
+template <int K, int SUBS, int TILES, int KW>
+void launch_gemm(const GemmArgs &a, hipStream_t stream) {
+    const dim3 grid((a.row_tiles + TILES - 1) / TILES, (a.tokens + SUBS * kSubTokens - 1) / (SUBS * kSubTokens));
+    q8_gemm_kernel<K, SUBS, TILES, KW><<<grid, KW * 64, 0, stream>>>(a);
+}
+
+// The split of a call: the tile shape with the least (rounds of one workgroup per CU) x
+// (2 SUBS + 1) x (TILES + 1), the last two for what a workgroup's step costs (its products,
+// and the loads of its fragments and codes), the smaller shape on a tie.  K goes over 8
+// waves, or over 4 where the large shapes fill the CUs more than once (two workgroups of 4
+// waves then share a CU).  Measured over 1 to 1024 tokens against every other shape, whole
+// calls: 5120 x 2880 at 16 tokens 2 tiles of 1 sub-tile 11.7 us (2 x 2 12.5), at 77 2 x 2 18.7
+// (4 x 5 24), at 128 2 x 5 19.5 (4 x 5 23.4), at 512 4 x 5 45.2 (4 x 3 58.8, 2 x 5 49.8); 2880 x
+// 4096 at 16 tokens 1 x 1 13.7, at 128 2 x 3 21.6 (2 x 2 27.7), at 512 4 x 3 49.2 (4 x 5, whose 288
+// workgroups are two rounds, 64.3).
+template <int K>
+void launch_gemm_for(const GemmArgs &a, uint32_t compute_units, hipStream_t stream) {
+    constexpr struct {
+        uint32_t subs, tiles;
+    } shapes[] = {{1, 1}, {1, 2}, {2, 2}, {2, 3}, {2, 5}, {4, 3}, {4, 5}};
+    const uint32_t subs = (a.tokens + kSubTokens - 1) / kSubTokens, cus = compute_units ? compute_units : 1;
+    uint64_t best = ~0ull;
+    uint32_t pick = 0, groups = 0;
+    for (uint32_t i = 0; i < 7; ++i) {
+        const uint32_t token_groups = (subs + shapes[i].subs - 1) / shapes[i].subs;
+        const uint64_t w = uint64_t((a.row_tiles + shapes[i].tiles - 1) / shapes[i].tiles) * token_groups;
+        const uint64_t cost = (w + cus - 1) / cus * (2 * shapes[i].subs + 1) * (shapes[i].tiles + 1);
+        if (cost < best && token_groups <= 65535u) {  // (the grid's y)
+            best = cost;
+            pick = i;
+            groups = w > cus ? 2 : 1;
+        }
+    }
+    switch (pick) {
+    case 0: launch_gemm<K, 1, 1, 8>(a, stream); break;
+    case 1: launch_gemm<K, 1, 2, 8>(a, stream); break;
+    case 2: launch_gemm<K, 2, 2, 8>(a, stream); break;
+    case 3: launch_gemm<K, 2, 3, 8>(a, stream); break;
+    case 4: groups > 1 ? launch_gemm<K, 2, 5, 4>(a, stream) : launch_gemm<K, 2, 5, 8>(a, stream); break;
+    case 5: groups > 1 ? launch_gemm<K, 4, 3, 4>(a, stream) : launch_gemm<K, 4, 3, 8>(a, stream); break;
+    default: groups > 1 ? launch_gemm<K, 4, 5, 4>(a, stream) : launch_gemm<K, 4, 5, 8>(a, stream); break;
+    }
+}
+
+template <int K>
+void launch_matmul(const GemmArgs &a, const float *x, bool shifted, int32_t *shift, uint8_t *frags,
+                   uint32_t compute_units, hipStream_t stream) {
+    const uint32_t gather = ((a.tokens + kSubTokens - 1) / kSubTokens) * (kSubTokens / kGatherWaves);
+    if (shifted) {
+        q8_gather_kernel<K, true><<<gather, kGatherWaves * 64, 0, stream>>>(x, a.tokens, shift, frags);
+    } else {
+        q8_gather_kernel<K, false><<<gather, kGatherWaves * 64, 0, stream>>>(x, a.tokens, shift, frags);
+    }
+    launch_gemm_for<K>(a, compute_units, stream);
 }
 
 int matmul_q8_0(ttl_ctx *ctx, const ttl_q8 *w, const float *bias_dev, const float *x_dev, const int32_t *shift_dev,
@@ -360,40 +423,27 @@ int matmul_q8_0(ttl_ctx *ctx, const ttl_q8 *w, const float *bias_dev, const floa
     if (tokens == 0) {
         return TTL_OK;
     }
-    const uint32_t tiles = (tokens + kTileTokens - 1) / kTileTokens;
+    uint8_t *frags = static_cast<uint8_t *>(workspace_dev);
+    int32_t *shift = shift_dev ? const_cast<int32_t *>(shift_dev)
+                               : reinterpret_cast<int32_t *>(frags + (w->cols == 2880 ? frag_bytes_for<2880>(tokens)
+                                                                                      : frag_bytes_for<4096>(tokens)));
     GemmArgs a;
     a.codes = w->codes;
     a.row_scales = w->row_scales;
     a.bias = bias_dev;
     a.residual = residual_dev;
     a.out = out_dev;
-    a.frags = static_cast<const uint8_t *>(workspace_dev);
-    int32_t *shift = reinterpret_cast<int32_t *>(static_cast<uint8_t *>(workspace_dev) +
-                                                 (w->cols == 2880 ? frag_bytes_for<2880>(tokens)
-                                                                  : frag_bytes_for<4096>(tokens)));
-    if (shift_dev) {
-        a.shift = shift_dev;
-    } else {
-        const int rc = ttl::launch_row_shifts(ctx->stream, x_dev, w->cols, tokens, w->cols, shift);
-        if (rc != TTL_OK) {
-            return rc;
-        }
-        a.shift = shift;
-    }
+    a.frags = frags;
+    a.shift = shift;
     a.rows = w->rows;
     a.row_tiles = w->tiles;
     a.tokens = tokens;
-    const uint32_t group = uint32_t(kWaves * kRowTiles);
-    const dim3 grid((w->tiles + group - 1) / group, tiles);
-    uint8_t *frags = static_cast<uint8_t *>(workspace_dev);
     if (w->cols == 2880) {
-        q8_gather_kernel<2880><<<dim3(Shape<2880>::steps, tiles), kSub * 64, 0, ctx->stream>>>(x_dev, tokens, a.shift,
-                                                                                               frags);
-        q8_gemm_kernel<2880><<<grid, kWaves * 64, 0, ctx->stream>>>(a);
+        launch_matmul<2880>(a, x_dev, shift_dev != nullptr, shift, frags, uint32_t(ctx->compute_units),
+                            ctx->stream);
     } else {
-        q8_gather_kernel<4096><<<dim3(Shape<4096>::steps, tiles), kSub * 64, 0, ctx->stream>>>(x_dev, tokens, a.shift,
-                                                                                               frags);
-        q8_gemm_kernel<4096><<<grid, kWaves * 64, 0, ctx->stream>>>(a);
+        launch_matmul<4096>(a, x_dev, shift_dev != nullptr, shift, frags, uint32_t(ctx->compute_units),
+                            ctx->stream);
     }
     TTL_LAUNCHED("q8 gemm kernels");
     return TTL_OK;
