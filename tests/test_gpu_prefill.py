@@ -144,6 +144,35 @@ def test_moe_prefill_experts_matches_oracle(dev, layer8, dtype):
         assert O.rel_l2(got[p], ref[p]) <= TOL, p
 
 
+# Buckets whose last tile is tiny (up to 16 slots), narrow (up to 32) or wide, at the edges
+# of each kind.  A token's result depends on no other token and its sums not on the kind of
+# its tile: a batch of the tokens at the buckets' ends alone gives the same bits.
+@pytest.mark.parametrize("dtype", [ttlab_amd.TTL_DTYPE_BF16, ttlab_amd.TTL_DTYPE_F32,
+                                   ttlab_amd.TTL_DTYPE_F32_AS_MXFP8])
+@pytest.mark.parametrize("buckets", [(1, 16, 17, 32, 33, 64, 65, 72), (15, 31, 48, 63, 81, 82, 0, 12)])
+def test_moe_prefill_tile_kinds(dev, layer8, dtype, buckets):
+    host, device = layer8
+    count = sum(buckets) // 4
+    rs = np.random.RandomState(sum(buckets))
+    left, idx = np.array(buckets), np.empty((count, 4), np.int32)
+    for p in rs.permutation(count):  # the four fullest experts left, so that each token's are distinct
+        idx[p] = rs.permutation(np.argsort(-left, kind="stable")[:4])
+        left[idx[p]] -= 1
+    assert not left.any()
+    w = rs.rand(count, 4).astype(np.float32)
+    x = O.synth_normal_bf16(0x78000002, 5, count * N, 1.0).reshape(count, N)
+    got = run_prefill(dev, device, x, idx, w, dtype)
+    ends = sorted({int(t[k]) for e in range(8) for t in [np.nonzero((idx == e).any(1))[0]] if t.size
+                   for k in (0, -1)})
+    alone = run_prefill(dev, device, x[ends], idx[ends], w[ends], dtype)
+    assert np.array_equal(got[ends].view(np.uint32), alone.view(np.uint32))
+    assert np.all(np.isfinite(got))
+    if dtype != ttlab_amd.TTL_DTYPE_F32_AS_MXFP8:
+        ref = oracle_prefill(host, x[ends], idx[ends], w[ends])
+        for p in range(len(ends)):
+            assert O.rel_l2(alone[p], ref[p]) <= TOL, ends[p]
+
+
 def test_moe_prefill_intermediates_exact_path(dev, layer8):
     """The exact path's stages read back per pair (ttl_moe_prefill_intermediates):
     the SwiGLU hidden against orc_swiglu of the oracle's gate and up, the down row

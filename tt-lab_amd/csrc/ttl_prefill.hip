@@ -58,19 +58,30 @@ constexpr int kMmRows = kMmWaves * kMmTiles * 16;
 constexpr int kHiddenPlanes = 3;
 
 // A tile holding at most kNarrowSlots slots (the remainder of an expert's bucket) is
-// "narrow": its GEMMs run on the first kNarrowCols column tiles only (a branch of the
-// same launch), so a bucket of 70 slots costs 64 + 32 columns instead of 64 + 64.
-constexpr int kNarrowCols = 2;
-constexpr uint32_t kNarrowSlots = kNarrowCols * 16;
+// "narrow", one of at most kTinySlots "tiny": its GEMMs run on, and its fragments are
+// written, staged and read for, the first kNarrowCols or kTinyCols column tiles only (a
+// branch of the same launch), so a bucket of 70 slots costs 64 + 16 columns instead of
+// 64 + 64.  A short prompt's buckets are all tiny (40 tokens over 128 experts: 1.7 slots
+// each) and its GEMMs bound by the weights: with 32 columns staged in 64-column stages they
+// ran at 3.2 and 2.7 TB/s (248 and 149 us), with the 16 they need at 4.3 TB/s (187 and 92).
+constexpr int kNarrowCols = 2, kTinyCols = 1;
+constexpr uint32_t kNarrowSlots = kNarrowCols * 16, kTinySlots = kTinyCols * 16;
 
 // ---- the plan ------------------------------------------------------------------
 
 struct PlanHeader {
     uint32_t tiles;    // token tiles in use
     uint32_t invalid;  // pairs whose expert index was out of range
-    uint32_t wide;     // tiles [0, wide) hold more than kNarrowSlots slots, [wide, tiles) at most that
-    uint32_t pad[61];
+    uint32_t wide;     // tiles [0, wide) hold more than kNarrowSlots slots,
+    uint32_t narrow;   // [wide, narrow) more than kTinySlots, [narrow, tiles) at most that
+    uint32_t pad[60];
 };
+
+// Column tiles of a tile that hold slots or may (the others are neither written nor read).
+__device__ inline uint32_t cols_of_tile(const PlanHeader *header, uint32_t tile) {
+    return tile < header->wide ? uint32_t(mf::col_tiles)
+                               : (tile < header->narrow ? uint32_t(kNarrowCols) : uint32_t(kTinyCols));
+}
 
 // Device pointers into the caller's workspace.
 struct Plan {
@@ -188,8 +199,7 @@ constexpr uint32_t kPlanPerLane = kMaxExperts / 64;  // experts per lane in the 
 __global__ __launch_bounds__(kPlanThreads) void plan_kernel(const int32_t *__restrict__ indices,
                                                             const float *__restrict__ weights, uint32_t pairs,
                                                             uint32_t used, uint32_t experts, Plan plan) {
-    __shared__ uint32_t count[kMaxExperts], base[kMaxExperts], running[kMaxExperts], narrow_of[kMaxExperts];
-    __shared__ uint32_t wide_total;
+    __shared__ uint32_t count[kMaxExperts], base[kMaxExperts], running[kMaxExperts], last_of[kMaxExperts];
     __shared__ uint32_t wave_count[kPlanThreads / 64][kMaxExperts];
     __shared__ uint32_t invalid;
     const uint32_t t = threadIdx.x, lane = t % 64, wave = t / 64;
@@ -234,41 +244,48 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(const int32_t *__res
     __syncthreads();
     if (wave == 0) {
         // wide tiles in expert order first, then the narrow ones (an expert's last tile
-        // when it holds at most kNarrowSlots slots), also in expert order: lane l takes
-        // experts kPlanPerLane l .. + kPlanPerLane - 1, and one prefix sum per quantity
-        // places them after the lanes before
-        uint32_t c[kPlanPerLane], slots = 0, wide = 0, narrow = 0;
+        // when it holds at most kNarrowSlots slots), then the tiny ones, also in expert
+        // order: lane l takes experts kPlanPerLane l .. + kPlanPerLane - 1, and one prefix
+        // sum per quantity places them after the lanes before
+        uint32_t c[kPlanPerLane], slots = 0, wide = 0, narrow = 0, tiny = 0;
+        const auto kind_of = [](uint32_t n) __attribute__((always_inline)) {  // of the last tile of n slots
+            const uint32_t rest = n - (n + mf::tile_slots - 1) / mf::tile_slots * mf::tile_slots + mf::tile_slots;
+            return n == 0 || rest > kNarrowSlots ? 0u : (rest > kTinySlots ? 1u : 2u);
+        };
 #pragma unroll
         for (uint32_t k = 0; k < kPlanPerLane; ++k) {
             const uint32_t e = lane * kPlanPerLane + k;
             c[k] = e < experts ? count[e] : 0u;
-            const uint32_t tiles = (c[k] + mf::tile_slots - 1) / mf::tile_slots;
-            const bool last_narrow = tiles > 0 && c[k] - (tiles - 1) * mf::tile_slots <= kNarrowSlots;
+            const uint32_t tiles = (c[k] + mf::tile_slots - 1) / mf::tile_slots, kind = kind_of(c[k]);
             slots += c[k];
-            wide += tiles - (last_narrow ? 1u : 0u);
-            narrow += last_narrow ? 1u : 0u;
+            wide += tiles - (kind ? 1u : 0u);
+            narrow += kind == 1u ? 1u : 0u;
+            tiny += kind == 2u ? 1u : 0u;
         }
         uint32_t s0 = wave_exclusive_sum(slots, lane), w0 = wave_exclusive_sum(wide, lane),
-                 n0 = wave_exclusive_sum(narrow, lane);
+                 n0 = wave_exclusive_sum(narrow, lane), t0 = wave_exclusive_sum(tiny, lane);
+        const uint32_t wide_total = __shfl(w0 + wide, 63), narrow_total = __shfl(n0 + narrow, 63);
+        n0 += wide_total;
+        t0 += wide_total + narrow_total;
+        if (lane == 63) {
+            plan.header->tiles = t0 + tiny;
+            plan.header->wide = wide_total;
+            plan.header->narrow = wide_total + narrow_total;
+            plan.header->invalid = invalid;
+        }
 #pragma unroll
         for (uint32_t k = 0; k < kPlanPerLane; ++k) {
             const uint32_t e = lane * kPlanPerLane + k;
-            const uint32_t tiles = (c[k] + mf::tile_slots - 1) / mf::tile_slots;
-            const bool last_narrow = tiles > 0 && c[k] - (tiles - 1) * mf::tile_slots <= kNarrowSlots;
+            const uint32_t tiles = (c[k] + mf::tile_slots - 1) / mf::tile_slots, kind = kind_of(c[k]);
             if (e < experts) {
                 base[e] = s0;
                 running[e] = w0;  // first wide tile of expert e (reset below)
-                narrow_of[e] = last_narrow ? n0 : ~0u;
+                last_of[e] = kind == 1u ? n0 : (kind == 2u ? t0 : ~0u);
             }
             s0 += c[k];
-            w0 += tiles - (last_narrow ? 1u : 0u);
-            n0 += last_narrow ? 1u : 0u;
-        }
-        if (lane == 63) {
-            wide_total = w0;
-            plan.header->tiles = w0 + n0;
-            plan.header->wide = w0;
-            plan.header->invalid = invalid;
+            w0 += tiles - (kind ? 1u : 0u);
+            n0 += kind == 1u ? 1u : 0u;
+            t0 += kind == 2u ? 1u : 0u;
         }
     }
     __syncthreads();
@@ -276,7 +293,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(const int32_t *__res
         const uint32_t n = count[e];
         for (uint32_t j = 0; j * mf::tile_slots < n; ++j) {
             const bool last = (j + 1) * mf::tile_slots >= n;
-            const uint32_t tile = last && narrow_of[e] != ~0u ? wide_total + narrow_of[e] : running[e] + j;
+            const uint32_t tile = last && last_of[e] != ~0u ? last_of[e] : running[e] + j;
             plan.tile_expert[tile] = e;
             plan.tile_first[tile] = base[e] + j * mf::tile_slots;
             plan.tile_count[tile] = min(uint32_t(mf::tile_slots), n - j * mf::tile_slots);
@@ -351,8 +368,10 @@ __global__ void plan_selected_kernel(const int32_t *__restrict__ tokens, uint32_
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t tiles = (count + mf::tile_slots - 1) / mf::tile_slots;
     if (i == 0) {
+        const uint32_t rest = count - (tiles - 1) * mf::tile_slots;  // the last tile's slots
         plan.header->tiles = tiles;
-        plan.header->wide = tiles;  // one launch over every tile
+        plan.header->wide = tiles - (rest <= kNarrowSlots ? 1u : 0u);
+        plan.header->narrow = tiles - (rest <= kTinySlots ? 1u : 0u);
         plan.header->invalid = 0;
     }
     if (i < tiles) {
@@ -425,6 +444,9 @@ __global__ __launch_bounds__(mf::col_tiles * 64) void gather_kernel(const void *
         return;
     }
     const uint32_t ct = threadIdx.x / 64, lane = threadIdx.x % 64;
+    if (ct >= cols_of_tile(plan.header, tile)) {
+        return;
+    }
     const uint32_t n = ct * 16 + lane % 16;
     const uint32_t block = quad * 4 + lane / 16;
     const bool block_ok = block < uint32_t(mx::blocks);
@@ -502,38 +524,36 @@ __global__ __launch_bounds__(mf::col_tiles * 64) void gather_kernel(const void *
 
 // ---- the MFMA main loop ----------------------------------------------------------------
 
-// K steps per LDS stage for P activation planes: a stage holds P * steps * 4
-// fragments (16 KiB for one plane, 24 KiB for three).
-template <int P>
+// K steps per LDS stage for P activation planes and NC column tiles: a stage holds
+// P * steps * NC fragments (16 KiB for one plane and four columns, 24 KiB for three planes).
+template <int P, int NC>
 struct StageShape {
-    static constexpr int steps = P == 1 ? 4 : 2;
+    static constexpr int steps = P * NC <= 4 ? 4 : 2;
     static constexpr int count = mf::steps / steps;
-    static constexpr int frags = P * steps * mf::col_tiles;
+    static constexpr int frags = P * steps * NC;
     static constexpr int chunks = frags * 64;  // 16-byte pieces
     static_assert(mf::steps % steps == 0, "stages must divide the K steps");
 };
 
-// Copies stage `j` of a token tile's fragments (P planes) between global memory
-// and LDS through registers; LDS order is [plane][step][column tile][lane].  Every
-// thread moves `per` pieces with no condition (a branch around a load makes the
-// compiler wait for it at once): pieces past the stage re-read its last piece and
-// land in the LDS buffer's padding.
-template <int P, int THREADS>
+// Copies stage `j` of a token tile's fragments (P planes, the first NC column tiles)
+// between global memory and LDS through registers; LDS order is [plane][step][column
+// tile][lane].  Every thread moves `per` pieces with no condition (a branch around a load
+// makes the compiler wait for it at once).
+template <int P, int THREADS, int NC>
 struct Stager {
-    using SS = StageShape<P>;
-    static constexpr int per = (SS::chunks + THREADS - 1) / THREADS;
-    static constexpr int lds_chunks = per * THREADS;  // LDS buffer size in pieces
+    using SS = StageShape<P, NC>;
+    static constexpr int per = SS::chunks / THREADS;
+    static_assert(SS::chunks % THREADS == 0, "whole pieces per thread");
     mf::u32x4 r[per];
 
     __device__ inline void load(const uint8_t *__restrict__ tile_frags, int j, uint32_t t) {
 #pragma unroll
         for (int k = 0; k < per; ++k) {
-            const uint32_t c = min(t + uint32_t(k) * THREADS, uint32_t(SS::chunks - 1));
-            const uint32_t plane = c / (SS::steps * mf::col_tiles * 64);
-            const uint32_t within = c % (SS::steps * mf::col_tiles * 64);
+            const uint32_t c = t + uint32_t(k) * THREADS;
+            const uint32_t row = c / (NC * 64), plane = row / SS::steps, step = row % SS::steps;
             r[k] = *reinterpret_cast<const mf::u32x4 *>(tile_frags + size_t(plane) * mf::plane_bytes +
-                                                    size_t(j) * SS::steps * mf::col_tiles * mf::frag_bytes +
-                                                    size_t(within) * 16);
+                                                    (size_t(j) * SS::steps + step) * mf::col_tiles * mf::frag_bytes +
+                                                    size_t(c % (NC * 64)) * 16);
         }
     }
     __device__ inline void store(mf::u32x4 *lds, uint32_t t) const {
@@ -543,6 +563,14 @@ struct Stager {
         }
     }
 };
+
+// 16-byte pieces of a stage buffer that serves wide, narrow and tiny tiles.
+template <int P>
+constexpr int stage_room() {
+    constexpr int a = StageShape<P, mf::col_tiles>::chunks, b = StageShape<P, kNarrowCols>::chunks,
+                  c = StageShape<P, kTinyCols>::chunks;
+    return a > b ? (a > c ? a : c) : (b > c ? b : c);
+}
 
 // One wave's A operand: NT 16-row tiles of repacked MXFP4 (ttl_internal.hpp), the
 // codes of one quad (4 K steps) per tile and the lane's 24 scale bytes per tile.
@@ -614,7 +642,7 @@ template <int P, int M, int LOOK, int NC, class V = bf16x8, class Decode, class 
 __device__ __attribute__((always_inline)) inline void quad_mfma(const mf::u32x4 *buf0, const mf::u32x4 *buf1,
                                                                 int i, uint32_t lane, Decode &&decode,
                                                                 StageEnd &&stage_end, f32x4 (&acc)[M][NC]) {
-    using SS = StageShape<P>;
+    using SS = StageShape<P, NC>;
     static_assert(NC >= 1 && NC <= mf::col_tiles, "column tiles");
     constexpr int FPS = P * NC;  // fragments per K step
     constexpr int SF = SS::steps * FPS;     // fragments per stage
@@ -625,7 +653,7 @@ __device__ __attribute__((always_inline)) inline void quad_mfma(const mf::u32x4 
         const mf::u32x4 *buf = (stage % 2) ? buf1 : buf0;
         auto frag = [&](int f) __attribute__((always_inline)) {
             const int ls = f / FPS, c = (f % FPS) / P, p = f % P;
-            return __builtin_bit_cast(V, buf[((p * SS::steps + ls) * mf::col_tiles + c) * 64 + lane]);
+            return __builtin_bit_cast(V, buf[((p * SS::steps + ls) * NC + c) * 64 + lane]);
         };
         V ring[D];
 #pragma unroll
@@ -699,20 +727,23 @@ __device__ inline bool tile_in_range(uint32_t tiles, uint32_t &tile, uint32_t &r
     return true;
 }
 
-// One launch covers every tile of the plan: the wide tiles [0, wide) run with all
-// mf::col_tiles column tiles, the narrow ones [wide, tiles) with kNarrowCols (the
+// A different empty statement for each instance of a template that a kernel branches to:
+// without it the compiler moves what the branches have in common (addresses, first loads)
+// in front of the branch, where it costs registers through all of them.
+#define TTL_OWN_CODE(NC) asm volatile("; %0 column tiles" ::"n"(NC))
+
+// One launch covers every tile of the plan, with the column tiles of its kind (the
 // workgroup's branch is uniform, so the barriers inside are reached by all its waves).
 __device__ inline bool tile_of_workgroup(const PlanHeader *header, uint32_t &tile, uint32_t &row_group,
-                                         bool &narrow) {
+                                         uint32_t &cols) {
     if (!tile_in_range(header->tiles, tile, row_group)) {
         return false;
     }
-    narrow = tile >= header->wide;
+    cols = cols_of_tile(header, tile);
     return true;
 }
 
-// Accumulators: [matrix (gate 0/1, up 2/3)][column tile]; NC column tiles (the plan's
-// wide tiles with all of them, or its narrow ones with kNarrowCols).
+// Accumulators: [matrix (gate 0/1, up 2/3)][column tile]; NC column tiles (by the tile's kind).
 // F16H: the hidden as two f16 planes of h x 2^kHiddenF16Shift (for the f16 down GEMM),
 // else three exact bf16 planes.  VX: the token operand, bf16x8 (PX exact planes; the
 // accumulators start at the bias) or f16x8 (two planes of x 2^k per column, k from
@@ -720,11 +751,11 @@ __device__ inline bool tile_of_workgroup(const PlanHeader *header, uint32_t &til
 // the sums are scaled back by 2^-k and the bias added before the SwiGLU.
 template <int PX, int NC, bool F16H, class VX>
 __device__ __attribute__((always_inline)) inline void gateup_tile(
-    const GateUpArgs &a, uint32_t tile, uint32_t row_group,
-    mf::u32x4 (*lds)[Stager<PX, kGuWaves * 64>::lds_chunks]) {
+    const GateUpArgs &a, uint32_t tile, uint32_t row_group, mf::u32x4 (*lds)[stage_room<PX>()]) {
     constexpr bool XS = __is_same(VX, mf::f16x8);
     static_assert(!XS || PX == 2, "f16 token operands are two planes");
-    using SS = StageShape<PX>;
+    using SS = StageShape<PX, NC>;
+    TTL_OWN_CODE(NC);
     constexpr int kThreads = kGuWaves * 64;
     const uint32_t t = threadIdx.x, wave = t / 64, lane = t % 64;
     const uint32_t expert = a.plan.tile_expert[tile];
@@ -771,7 +802,7 @@ __device__ __attribute__((always_inline)) inline void gateup_tile(
         }
     }
 
-    Stager<PX, kThreads> st;
+    Stager<PX, kThreads, NC> st;
     st.load(frags, 0, t);
     // three planes leave room for one code buffer less (the fourth spilled)
     constexpr int NB = PX == 3 ? 3 : kGuCodeBuffers;
@@ -882,13 +913,14 @@ __device__ __attribute__((always_inline)) inline void gateup_tile(
 
 template <int PX, bool F16H, class VX = bf16x8>
 __global__ __launch_bounds__(kGuWaves * 64) __attribute__((amdgpu_waves_per_eu(2))) void gateup_kernel(GateUpArgs a) {
-    __shared__ mf::u32x4 lds[2][Stager<PX, kGuWaves * 64>::lds_chunks];
-    uint32_t tile, row_group;
-    bool narrow;
-    if (!tile_of_workgroup(a.plan.header, tile, row_group, narrow)) {
+    __shared__ mf::u32x4 lds[2][stage_room<PX>()];
+    uint32_t tile, row_group, cols;
+    if (!tile_of_workgroup(a.plan.header, tile, row_group, cols)) {
         return;
     }
-    if (narrow) {
+    if (cols == uint32_t(kTinyCols)) {
+        gateup_tile<PX, kTinyCols, F16H, VX>(a, tile, row_group, lds);
+    } else if (cols == uint32_t(kNarrowCols)) {
         gateup_tile<PX, kNarrowCols, F16H, VX>(a, tile, row_group, lds);
     } else {
         gateup_tile<PX, mf::col_tiles, F16H, VX>(a, tile, row_group, lds);
@@ -914,8 +946,9 @@ struct MatmulArgs {
 template <int P, bool SCATTER, int NC, class V, int SHIFT>
 __device__ __attribute__((always_inline)) inline void matmul_tile(const MatmulArgs &a, uint32_t tile,
                                                                   uint32_t row_group,
-                                                                  mf::u32x4 (*lds)[Stager<P, kMmWaves * 64>::lds_chunks]) {
-    using SS = StageShape<P>;
+                                                                  mf::u32x4 (*lds)[stage_room<P>()]) {
+    using SS = StageShape<P, NC>;
+    TTL_OWN_CODE(NC);
     constexpr int kThreads = kMmWaves * 64;
     const uint32_t t = threadIdx.x, wave = t / 64, lane = t % 64;
     const uint32_t expert = a.plan.tile_expert[tile];
@@ -957,7 +990,7 @@ __device__ __attribute__((always_inline)) inline void matmul_tile(const MatmulAr
         }
     }
 
-    Stager<P, kThreads> st;
+    Stager<P, kThreads, NC> st;
     st.load(frags, 0, t);
     uint4 qa[3][kMmTiles];
     wa.load(0, lane, qa[0]);
@@ -1049,13 +1082,14 @@ __device__ __attribute__((always_inline)) inline void matmul_tile(const MatmulAr
 
 template <int P, bool SCATTER, class V = bf16x8, int SHIFT = 0>
 __global__ __launch_bounds__(kMmWaves * 64) void matmul_kernel(MatmulArgs a) {
-    __shared__ mf::u32x4 lds[2][Stager<P, kMmWaves * 64>::lds_chunks];
-    uint32_t tile, row_group;
-    bool narrow;
-    if (!tile_of_workgroup(a.plan.header, tile, row_group, narrow)) {
+    __shared__ mf::u32x4 lds[2][stage_room<P>()];
+    uint32_t tile, row_group, cols;
+    if (!tile_of_workgroup(a.plan.header, tile, row_group, cols)) {
         return;
     }
-    if (narrow) {
+    if (cols == uint32_t(kTinyCols)) {
+        matmul_tile<P, SCATTER, kTinyCols, V, SHIFT>(a, tile, row_group, lds);
+    } else if (cols == uint32_t(kNarrowCols)) {
         matmul_tile<P, SCATTER, kNarrowCols, V, SHIFT>(a, tile, row_group, lds);
     } else {
         matmul_tile<P, SCATTER, mf::col_tiles, V, SHIFT>(a, tile, row_group, lds);
@@ -1118,6 +1152,9 @@ __global__ __launch_bounds__(256) void gather_mx8_kernel(const void *__restrict_
         return;
     }
     const uint32_t quad = blockIdx.x / mf::col_tiles, ct = blockIdx.x % mf::col_tiles;
+    if (ct >= cols_of_tile(plan.header, tile)) {
+        return;
+    }
     const uint32_t t = threadIdx.x, n16 = t / 16, g = (t % 16) / 4, r = t % 4;
     const uint32_t n = ct * 16 + n16, block = 4 * quad + g;
     const bool block_ok = block < uint32_t(mx::blocks);
@@ -1188,9 +1225,9 @@ __global__ __launch_bounds__(256) void gather_mx8_kernel(const void *__restrict_
 constexpr int kMx8StageQuads = 2;
 constexpr size_t kMx8StageBytes = size_t(kMx8StageQuads) * mf::col_tiles * mx8::frag_bytes;  // 16 KiB
 
-template <int THREADS>
+template <int THREADS, int NC>
 struct Mx8Stager {
-    static constexpr int pieces = int(kMx8StageBytes / 16);
+    static constexpr int pieces = kMx8StageQuads * NC * int(mx8::frag_bytes / 16);  // of the first NC column tiles
     static constexpr int per = pieces / THREADS;
     static_assert(pieces % THREADS == 0, "whole pieces per thread");
     mf::u32x4 r[per];
@@ -1199,7 +1236,10 @@ struct Mx8Stager {
     __device__ inline void load(const uint8_t *__restrict__ tile_frags, int stage, uint32_t t) {
 #pragma unroll
         for (int k = 0; k < per; ++k) {
-            const size_t off = min(size_t(stage) * kMx8StageBytes + (size_t(t) + size_t(k) * THREADS) * 16,
+            constexpr uint32_t row = NC * uint32_t(mx8::frag_bytes / 16);  // pieces of a quad
+            const uint32_t piece = t + uint32_t(k) * THREADS;
+            const size_t off = min(size_t(stage) * kMx8StageBytes + piece / row * (mf::col_tiles * mx8::frag_bytes) +
+                                       size_t(piece % row) * 16,
                                    mx8::tile_frag_bytes - 16);
             r[k] = *reinterpret_cast<const mf::u32x4 *>(tile_frags + off);
         }
@@ -1227,12 +1267,12 @@ struct Mx8Stager {
 // around a load: the compiler would wait for it at once).
 template <int M, int NC, int THREADS>
 __device__ __attribute__((always_inline)) inline void mx8_quad(int i, uint4 (&q)[M], int next, AOperand<M> &wa,
-                                                               uint32_t (&sb)[NC][6], Mx8Stager<THREADS> &st,
+                                                               uint32_t (&sb)[NC][6], Mx8Stager<THREADS, NC> &st,
                                                                const uint8_t *tile_frags,
                                                                mf::u32x4 (*lds)[kMx8StageBytes / 16], uint32_t t,
                                                                uint32_t lane, mf::f32x4 (&acc)[M][NC], bool stage_end) {
     const int stage = i / kMx8StageQuads;
-    const mf::u32x4 *buf = lds[stage % 2] + size_t(i % kMx8StageQuads) * mf::col_tiles * 64 * 2;
+    const mf::u32x4 *buf = lds[stage % 2] + size_t(i % kMx8StageQuads) * NC * 64 * 2;
     mx8::i32x8 b[NC];
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
@@ -1303,7 +1343,7 @@ __device__ __attribute__((always_inline)) inline void mx8_main_loop(AOperand<M> 
         sb[c][4] = r2.x;
         sb[c][5] = r2.y;
     }
-    Mx8Stager<THREADS> st;
+    Mx8Stager<THREADS, NC> st;
     st.load(tile_frags, 0, t);
     uint4 q[2][M];
     wa.load(0, lane, q[0]);
@@ -1329,6 +1369,7 @@ template <int NC>
 __device__ __attribute__((always_inline)) inline void mx8_gateup_tile(const GateUpArgs &a, uint32_t tile,
                                                                       uint32_t row_group,
                                                                       mf::u32x4 (*lds)[kMx8StageBytes / 16]) {
+    TTL_OWN_CODE(NC);
     constexpr int kThreads = kGuWaves * 64;
     const uint32_t t = threadIdx.x, wave = t / 64, lane = t % 64;
     const uint32_t expert = a.plan.tile_expert[tile];
@@ -1431,12 +1472,13 @@ __device__ __attribute__((always_inline)) inline void mx8_gateup_tile(const Gate
 
 __global__ __launch_bounds__(kGuWaves * 64) void mx8_gateup_kernel(GateUpArgs a) {
     __shared__ mf::u32x4 lds[2][kMx8StageBytes / 16];
-    uint32_t tile, row_group;
-    bool narrow;
-    if (!tile_of_workgroup(a.plan.header, tile, row_group, narrow)) {
+    uint32_t tile, row_group, cols;
+    if (!tile_of_workgroup(a.plan.header, tile, row_group, cols)) {
         return;
     }
-    if (narrow) {
+    if (cols == uint32_t(kTinyCols)) {
+        mx8_gateup_tile<kTinyCols>(a, tile, row_group, lds);
+    } else if (cols == uint32_t(kNarrowCols)) {
         mx8_gateup_tile<kNarrowCols>(a, tile, row_group, lds);
     } else {
         mx8_gateup_tile<mf::col_tiles>(a, tile, row_group, lds);
@@ -1449,6 +1491,7 @@ template <bool SCATTER, int NC>
 __device__ __attribute__((always_inline)) inline void mx8_matmul_tile(const MatmulArgs &a, uint32_t tile,
                                                                       uint32_t row_group,
                                                                       mf::u32x4 (*lds)[kMx8StageBytes / 16]) {
+    TTL_OWN_CODE(NC);
     constexpr int kThreads = kMmWaves * 64;
     const uint32_t t = threadIdx.x, wave = t / 64, lane = t % 64;
     const uint32_t expert = a.plan.tile_expert[tile];
@@ -1515,12 +1558,13 @@ __device__ __attribute__((always_inline)) inline void mx8_matmul_tile(const Matm
 template <bool SCATTER>
 __global__ __launch_bounds__(kMmWaves * 64) void mx8_matmul_kernel(MatmulArgs a) {
     __shared__ mf::u32x4 lds[2][kMx8StageBytes / 16];
-    uint32_t tile, row_group;
-    bool narrow;
-    if (!tile_of_workgroup(a.plan.header, tile, row_group, narrow)) {
+    uint32_t tile, row_group, cols;
+    if (!tile_of_workgroup(a.plan.header, tile, row_group, cols)) {
         return;
     }
-    if (narrow) {
+    if (cols == uint32_t(kTinyCols)) {
+        mx8_matmul_tile<SCATTER, kTinyCols>(a, tile, row_group, lds);
+    } else if (cols == uint32_t(kNarrowCols)) {
         mx8_matmul_tile<SCATTER, kNarrowCols>(a, tile, row_group, lds);
     } else {
         mx8_matmul_tile<SCATTER, mf::col_tiles>(a, tile, row_group, lds);
@@ -1991,7 +2035,7 @@ int moe_prefill_run(ttl_ctx *ctx, const ttl_moe_layer *layer, const void *x_dev,
     g.rows = L.expert_hidden;
     g.tiles_per_expert = L.gate->tiles;
     g.plan = plan;
-    // one launch per GEMM over the wide tiles and the narrow ones (at most one per expert)
+    // one launch per GEMM over the wide tiles and the narrow and tiny ones (at most one per expert)
     const dim3 gu_grid((L.expert_hidden + kGuRows - 1) / kGuRows, lay.tmax);
     if ((stages & TTL_PREFILL_GATEUP) && scaled) {
         mx8_gateup_kernel<<<gu_grid, kGuWaves * 64, 0, ctx->stream>>>(g);
