@@ -572,6 +572,51 @@ constexpr int stage_room() {
     return a > b ? (a > c ? a : c) : (b > c ? b : c);
 }
 
+// The stages of one tile's GEMM in the order of its weight requests.  Loads return in order,
+// so a wave that waits for a stage's pieces also waits for every weight request before
+// them.  Wide and narrow tiles request a stage two stages ahead (more does not fit their
+// registers); a tiny tile, whose stage is a quad and two registers quads of pieces, requests
+// it with that quad's codes, NB - 1 quads ahead, and so keeps that many quads of weights in
+// flight.  (40 tokens over 32 experts, whole layer: one stage ahead 143 us, with the codes
+// 138; 50 tokens, experts alone, f32 117.7 and 112.5, bf16 104.4 and 100.0.)
+template <int P, int THREADS, int NC, int NB>
+struct StageRing {
+    using SS = StageShape<P, NC>;
+    static constexpr bool deep = NC == kTinyCols;
+    static_assert(!deep || SS::steps == 4, "a tiny tile's stage is one quad");
+    Stager<P, THREADS, NC> s[deep ? NB : 1];
+
+    __device__ inline void begin(const uint8_t *frags, uint32_t t) {
+        if (!deep) {
+            s[0].load(frags, 0, t);
+        }
+    }
+    // called with the request of quad i's codes into buffer b
+    __device__ inline void with_codes(const uint8_t *frags, int i, int b, uint32_t t) {
+        if (deep) {
+            s[deep ? b : 0].load(frags, i, t);
+        }
+    }
+    __device__ inline void first(const uint8_t *frags, mf::u32x4 (*lds)[stage_room<P>()], uint32_t t) {
+        s[0].store(lds[0], t);
+        __syncthreads();
+        if (!deep && SS::count > 1) {
+            s[0].load(frags, 1, t);
+        }
+    }
+    // end of stage (a quad in buffer b for a tiny tile): publish the next, fetch ahead
+    __device__ inline void next(const uint8_t *frags, int stage, int b, mf::u32x4 (*lds)[stage_room<P>()], uint32_t t) {
+        if (stage + 1 < SS::count) {
+            s[deep ? (b + 1) % NB : 0].store(lds[(stage + 1) % 2], t);
+        }
+        __syncthreads();
+        if (!deep && stage + 2 < SS::count) {
+            s[0].load(frags, stage + 2, t);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+};
+
 // One wave's A operand: NT 16-row tiles of repacked MXFP4 (ttl_internal.hpp), the
 // codes of one quad (4 K steps) per tile and the lane's 24 scale bytes per tile.
 template <int NT>
@@ -685,7 +730,8 @@ __device__ __attribute__((always_inline)) inline void quad_mfma(const mf::u32x4 
 // it).  The caller has requested quads 0..NB-2 into buffers 0..NB-2.  Each request
 // is pinned before the quad's instructions (sched_barrier), and so are the stage
 // requests at every stage end: left to the scheduler, requests sank to just before
-// their first use and the wave waited for them there.
+// their first use and the wave waited for them there.  load and compute are told the
+// buffer's number too (a constant after unrolling).
 template <int NB, int M, class Load, class Compute>
 __device__ __attribute__((always_inline)) inline void rotate_quads(uint4 (&qa)[NB][M], Load &&load,
                                                                    Compute &&compute) {
@@ -693,9 +739,9 @@ __device__ __attribute__((always_inline)) inline void rotate_quads(uint4 (&qa)[N
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
             if (i + b < mf::quads) {
-                load(min(i + b + NB - 1, mf::quads - 1), qa[(b + NB - 1) % NB]);
+                load(min(i + b + NB - 1, mf::quads - 1), qa[(b + NB - 1) % NB], (b + NB - 1) % NB);
                 __builtin_amdgcn_sched_barrier(0);
-                compute(i + b, qa[b]);
+                compute(i + b, qa[b], b);
             }
         }
     }
@@ -754,7 +800,6 @@ __device__ __attribute__((always_inline)) inline void gateup_tile(
     const GateUpArgs &a, uint32_t tile, uint32_t row_group, mf::u32x4 (*lds)[stage_room<PX>()]) {
     constexpr bool XS = __is_same(VX, mf::f16x8);
     static_assert(!XS || PX == 2, "f16 token operands are two planes");
-    using SS = StageShape<PX, NC>;
     TTL_OWN_CODE(NC);
     constexpr int kThreads = kGuWaves * 64;
     const uint32_t t = threadIdx.x, wave = t / 64, lane = t % 64;
@@ -802,12 +847,13 @@ __device__ __attribute__((always_inline)) inline void gateup_tile(
         }
     }
 
-    Stager<PX, kThreads, NC> st;
-    st.load(frags, 0, t);
     // three planes leave room for one code buffer less (the fourth spilled)
     constexpr int NB = PX == 3 ? 3 : kGuCodeBuffers;
+    using Stages = StageRing<PX, kThreads, NC, NB>;
+    Stages st;
     uint4 qa[NB][4];  // codes of the quads in flight: [buffer][gate0, gate1, up0, up1]
-    auto load_quad = [&](int i, uint4(&q)[4]) __attribute__((always_inline)) {
+    auto load_quad = [&](int i, uint4(&q)[4], int b) __attribute__((always_inline)) {
+        st.with_codes(frags, i, b, t);
         uint4 g2[2], u2[2];
         ga.load(i, lane, g2);
         ua.load(i, lane, u2);
@@ -816,28 +862,14 @@ __device__ __attribute__((always_inline)) inline void gateup_tile(
         q[2] = u2[0];
         q[3] = u2[1];
     };
+    st.begin(frags, t);
 #pragma unroll
     for (int b = 0; b < NB - 1; ++b) {
-        load_quad(b, qa[b]);
+        load_quad(b, qa[b], b);
     }
-    st.store(lds[0], t);
-    __syncthreads();
-    if (SS::count > 1) {
-        st.load(frags, 1, t);
-    }
+    st.first(frags, lds, t);
 
-    auto stage_end = [&](int stage) __attribute__((always_inline)) {
-        // end of stage: publish the next stage, fetch the one after
-        if (stage + 1 < SS::count) {
-            st.store(lds[(stage + 1) % 2], t);
-        }
-        __syncthreads();
-        if (stage + 2 < SS::count) {
-            st.load(frags, stage + 2, t);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    auto compute_quad = [&](int i, const uint4(&q)[4]) __attribute__((always_inline)) {
+    auto compute_quad = [&](int i, const uint4(&q)[4], int b) __attribute__((always_inline)) {
         float sc[4];
         sc[0] = ga.scale(0);
         sc[1] = ga.scale(1);
@@ -854,6 +886,7 @@ __device__ __attribute__((always_inline)) inline void gateup_tile(
         };
         // B fragments four ahead of their MFMAs for one plane and for three (with three
         // planes this fits the 256 registers of two waves per SIMD without spilling)
+        auto stage_end = [&](int stage) __attribute__((always_inline)) { st.next(frags, stage, b, lds, t); };
         quad_mfma<PX, 4, 4, NC, VX>(lds[0], lds[1], i, lane, decode, stage_end, acc);
     };
 
@@ -947,7 +980,6 @@ template <int P, bool SCATTER, int NC, class V, int SHIFT>
 __device__ __attribute__((always_inline)) inline void matmul_tile(const MatmulArgs &a, uint32_t tile,
                                                                   uint32_t row_group,
                                                                   mf::u32x4 (*lds)[stage_room<P>()]) {
-    using SS = StageShape<P, NC>;
     TTL_OWN_CODE(NC);
     constexpr int kThreads = kMmWaves * 64;
     const uint32_t t = threadIdx.x, wave = t / 64, lane = t % 64;
@@ -990,28 +1022,22 @@ __device__ __attribute__((always_inline)) inline void matmul_tile(const MatmulAr
         }
     }
 
-    Stager<P, kThreads, NC> st;
-    st.load(frags, 0, t);
-    uint4 qa[3][kMmTiles];
-    wa.load(0, lane, qa[0]);
-    wa.load(1, lane, qa[1]);
-    st.store(lds[0], t);
-    __syncthreads();
-    if (SS::count > 1) {
-        st.load(frags, 1, t);
-    }
-
-    auto stage_end = [&](int stage) __attribute__((always_inline)) {
-        if (stage + 1 < SS::count) {
-            st.store(lds[(stage + 1) % 2], t);
-        }
-        __syncthreads();
-        if (stage + 2 < SS::count) {
-            st.load(frags, stage + 2, t);
-        }
-        __builtin_amdgcn_sched_barrier(0);
+    constexpr int NB = NC == kTinyCols ? 4 : 3;  // code buffers
+    using Stages = StageRing<P, kThreads, NC, NB>;
+    Stages st;
+    uint4 qa[NB][kMmTiles];
+    auto load_quad = [&](int i, uint4(&q)[kMmTiles], int b) __attribute__((always_inline)) {
+        st.with_codes(frags, i, b, t);
+        wa.load(i, lane, q);
     };
-    auto compute_quad = [&](int i, const uint4(&q)[kMmTiles]) __attribute__((always_inline)) {
+    st.begin(frags, t);
+#pragma unroll
+    for (int b = 0; b < NB - 1; ++b) {
+        load_quad(b, qa[b], b);
+    }
+    st.first(frags, lds, t);
+
+    auto compute_quad = [&](int i, const uint4(&q)[kMmTiles], int b) __attribute__((always_inline)) {
         float sc[kMmTiles];
 #pragma unroll
         for (int m = 0; m < kMmTiles; ++m) {
@@ -1025,24 +1051,11 @@ __device__ __attribute__((always_inline)) inline void matmul_tile(const MatmulAr
                 w[m] = mf::decode_as<V>(word, sc[m]);
             }
         };
+        auto stage_end = [&](int stage) __attribute__((always_inline)) { st.next(frags, stage, b, lds, t); };
         quad_mfma<P, kMmTiles, 4, NC, V>(lds[0], lds[1], i, lane, decode, stage_end, acc);
     };
 
-    for (int i = 0; i < mf::quads; i += 3) {
-        wa.load(min(i + 2, mf::quads - 1), lane, qa[2]);
-        __builtin_amdgcn_sched_barrier(0);
-        compute_quad(i, qa[0]);
-        wa.load(min(i + 3, mf::quads - 1), lane, qa[0]);
-        __builtin_amdgcn_sched_barrier(0);
-        if (i + 1 < mf::quads) {
-            compute_quad(i + 1, qa[1]);
-            wa.load(min(i + 4, mf::quads - 1), lane, qa[1]);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        if (i + 2 < mf::quads) {
-            compute_quad(i + 2, qa[2]);
-        }
-    }
+    rotate_quads(qa, load_quad, compute_quad);
 
     if (!rows_ok) {
         return;
