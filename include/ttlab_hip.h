@@ -60,6 +60,14 @@ int ttl_free(ttl_ctx *ctx, void *dev);
 int ttl_memcpy_h2d(ttl_ctx *ctx, void *dst_dev, const void *src, size_t bytes);
 int ttl_memcpy_d2h(ttl_ctx *ctx, void *dst, const void *src_dev, size_t bytes);
 int ttl_memcpy_d2d(ttl_ctx *ctx, void *dst_dev, const void *src_dev, size_t bytes);
+/* Page-locked host memory, for ttl_memcpy_d2h of what a caller reads after every step: the
+ * copy is one DMA, where pageable memory goes through the runtime's staging buffer.  Any
+ * context's copies may use it. */
+int ttl_host_malloc(ttl_ctx *ctx, size_t bytes, void **host);
+int ttl_host_free(ttl_ctx *ctx, void *host);
+/* dst_dev[0 .. count) = words, count <= 4, by a launch that carries the words: stream-ordered,
+ * with no copy and no wait (ttl_memcpy_h2d waits for the stream).  dst_dev 4-byte aligned. */
+int ttl_set_words(ttl_ctx *ctx, uint32_t *dst_dev, const uint32_t *words, uint32_t count);
 /* Fills with a byte value using a kernel (safe inside HIP graph capture). */
 int ttl_fill_bytes(ttl_ctx *ctx, void *dst_dev, uint8_t value, size_t bytes);
 

@@ -40,3 +40,29 @@ def test_stream_read_reads_every_load(words):
     src.free()
     sink.free()
     dev.close()
+
+
+@pytest.mark.parametrize("count", [0, 1, 3, 4])
+def test_set_words_and_host_memory(count):
+    """ttl_set_words writes exactly `count` words, in stream order with copies around it; a
+    page-locked buffer takes a device copy."""
+    import ctypes as C
+    import ttlab_amd
+    dev = ttlab_amd.Device(0)
+    try:
+        buf = dev.upload(np.arange(6, dtype=np.uint32))
+        words = np.array([0xfffffff0 + i for i in range(4)], np.uint32)
+        ttlab_amd._check(dev.lib.ttl_set_words(dev.ctx, buf.ptr + 4, words.ctypes.data, count), "ttl_set_words")
+        words[:] = 1  # the launch holds the values
+        host = C.c_void_p()
+        ttlab_amd._check(dev.lib.ttl_host_malloc(dev.ctx, 24, C.byref(host)), "ttl_host_malloc")
+        ttlab_amd._check(dev.lib.ttl_memcpy_d2h(dev.ctx, host, buf.ptr, 24), "ttl_memcpy_d2h")
+        got = np.ctypeslib.as_array(C.cast(host, C.POINTER(C.c_uint32)), (6,)).copy()
+        ttlab_amd._check(dev.lib.ttl_host_free(dev.ctx, host), "ttl_host_free")
+        expect = np.arange(6, dtype=np.uint32)
+        expect[1:1 + count] = [0xfffffff0 + i for i in range(count)]
+        assert np.array_equal(got, expect)
+        assert dev.lib.ttl_set_words(dev.ctx, buf.ptr, words.ctypes.data, 5) == -2
+        buf.free()
+    finally:
+        dev.close()

@@ -17,6 +17,16 @@ __global__ void fill_bytes_kernel(uint8_t *dst, uint8_t value, size_t n) {
     }
 }
 
+__global__ void set_words_kernel(uint32_t *dst, uint4 words, uint32_t count) {
+    const uint32_t w[4] = {words.x, words.y, words.z, words.w};
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) {
+        if (i < count) {
+            dst[i] = w[i];
+        }
+    }
+}
+
 // 16-byte vector copy, grid-stride: the known-size reference dispatch for the byte
 // counters (each byte read once and written once).
 __global__ void copy16_kernel(const uint4 *__restrict__ src, uint4 *__restrict__ dst, size_t n) {
@@ -419,6 +429,38 @@ int ttl_memcpy_d2d(ttl_ctx *ctx, void *dst_dev, const void *src_dev, size_t byte
     const unsigned blocks = unsigned(std::min<size_t>(ttl::blocks_for(n, threads), 8192));
     copy16_kernel<<<blocks, threads, 0, ctx->stream>>>((const uint4 *)src_dev, (uint4 *)dst_dev, n);
     TTL_LAUNCHED("copy16_kernel");
+    return TTL_OK;
+}
+
+int ttl_host_malloc(ttl_ctx *ctx, size_t bytes, void **host) {
+    TTL_REQUIRE(ctx && host, TTL_ERR_INVALID, "ttl_host_malloc: null argument");
+    *host = nullptr;
+    TTL_HIP(hipSetDevice(ctx->device));
+    TTL_HIP(hipHostMalloc(host, bytes ? bytes : 1, hipHostMallocDefault));
+    return TTL_OK;
+}
+
+int ttl_host_free(ttl_ctx *ctx, void *host) {
+    TTL_REQUIRE(ctx, TTL_ERR_INVALID, "ttl_host_free: null context");
+    if (host) {
+        TTL_HIP(hipStreamSynchronize(ctx->stream));
+        TTL_HIP(hipHostFree(host));
+    }
+    return TTL_OK;
+}
+
+int ttl_set_words(ttl_ctx *ctx, uint32_t *dst_dev, const uint32_t *words, uint32_t count) {
+    TTL_REQUIRE(ctx && (count == 0 || (dst_dev && words)), TTL_ERR_INVALID, "ttl_set_words: null argument");
+    TTL_REQUIRE(count <= 4, TTL_ERR_SHAPE, "ttl_set_words: at most 4 words");
+    TTL_REQUIRE((reinterpret_cast<uintptr_t>(dst_dev) & 3) == 0, TTL_ERR_INVALID,
+                "ttl_set_words: the destination must be 4-byte aligned");
+    if (count == 0) {
+        return TTL_OK;
+    }
+    uint32_t w[4] = {};
+    std::memcpy(w, words, sizeof(uint32_t) * count);
+    set_words_kernel<<<1, 1, 0, ctx->stream>>>(dst_dev, make_uint4(w[0], w[1], w[2], w[3]), count);
+    TTL_LAUNCHED("set_words_kernel");
     return TTL_OK;
 }
 

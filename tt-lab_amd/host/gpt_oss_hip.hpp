@@ -222,7 +222,7 @@ class HipGptOssModel {
     void *logits_workspace_ = nullptr;
     ttl_graph *step_ = nullptr;
     bool use_graph_ = true;
-    std::vector<float> host_logits_;
+    float *host_logits_ = nullptr;  // page-locked: forward and prefill copy the logits there
     // layer-major prefill (model.cpp:463-555), chunks of prefill_batch_ tokens
     size_t prefill_batch_ = 0;
     bool prefill_by_decode_ = false;  // some expert tensor has E8M0 scale 0 or 255

@@ -334,6 +334,9 @@ def load_library():
         "ttl_memcpy_h2d": (i32, [vp, vp, vp, sz]),
         "ttl_memcpy_d2h": (i32, [vp, vp, vp, sz]),
         "ttl_memcpy_d2d": (i32, [vp, vp, vp, sz]),
+        "ttl_host_malloc": (i32, [vp, sz, C.POINTER(vp)]),
+        "ttl_host_free": (i32, [vp, vp]),
+        "ttl_set_words": (i32, [vp, vp, vp, u32]),
         "ttl_fill_bytes": (i32, [vp, vp, C.c_uint8, sz]),
         "ttl_timer_start": (i32, [vp]),
         "ttl_timer_stop": (i32, [vp, C.POINTER(f32)]),
