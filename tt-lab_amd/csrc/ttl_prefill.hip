@@ -756,37 +756,50 @@ struct GateUpArgs {
     Plan plan;
 };
 
-// Workgroup -> (token tile, row group).  Workgroups are dispatched round-robin
-// over the chip's 8 XCDs (each with its own L2), so consecutive logical indices
-// are taken from the same XCD: all row groups of one token tile then read its
-// activation fragments through one L2.  Workgroups past the tiles in use return.
-__device__ inline bool tile_in_range(uint32_t tiles, uint32_t &tile, uint32_t &row_group) {
-    const uint32_t groups = gridDim.x;
-    const uint32_t id = blockIdx.y * groups + blockIdx.x;
-    const uint32_t active = tiles * groups;
-    if (id >= active) {
-        return false;
-    }
-    const uint32_t logical = active % 8 == 0 ? (id % 8) * (active / 8) + id / 8 : id;
-    tile = logical / groups;
-    row_group = logical % groups;
-    return true;
-}
-
 // A different empty statement for each instance of a template that a kernel branches to:
 // without it the compiler moves what the branches have in common (addresses, first loads)
 // in front of the branch, where it costs registers through all of them.
 #define TTL_OWN_CODE(NC) asm volatile("; %0 column tiles" ::"n"(NC))
 
-// One launch covers every tile of the plan, with the column tiles of its kind (the
-// workgroup's branch is uniform, so the barriers inside are reached by all its waves).
+// Workgroup -> (token tile, row group) and the tile's column tiles; one launch covers every
+// tile of the plan (the workgroup's branch on its kind is uniform, so the barriers inside are
+// reached by all its waves).  Workgroups are dealt to the chip's 8 XCDs in turn, each with
+// its own L2 and its own queue: XCD k takes an eighth of the wide tiles' workgroups, then an
+// eighth of the narrow ones', then of the tiny ones', each eighth consecutive, so that all row
+// groups of one token tile read its activation fragments through one L2 and every XCD has as
+// much of each kind as the others.  (With one list cut in eight, wide tiles first, the XCDs
+// of the last eighths had only small tiles: the MoE layer of 512 tokens over 32 experts
+// 289 us, of 200 tokens 217; this way 273 and 178.  The wide workgroups of a last, partly
+// filled round as two halves of their columns: 285 and 182, a half takes nearly as long.)
+// Workgroups past an XCD's share return; xcd_grid() launches enough for every share.
+constexpr uint32_t kXcds = 8;
+
 __device__ inline bool tile_of_workgroup(const PlanHeader *header, uint32_t &tile, uint32_t &row_group,
                                          uint32_t &cols) {
-    if (!tile_in_range(header->tiles, tile, row_group)) {
-        return false;
+    const uint32_t groups = gridDim.x, id = blockIdx.y * groups + blockIdx.x;
+    const uint32_t xcd = id % kXcds;
+    const uint32_t bound[4] = {0, header->wide, header->narrow, header->tiles};
+    uint32_t place = id / kXcds;
+#pragma unroll
+    for (int kind = 0; kind < 3; ++kind) {
+        const uint32_t work = (bound[kind + 1] - bound[kind]) * groups;
+        const uint32_t first = uint32_t(uint64_t(work) * xcd / kXcds);
+        const uint32_t share = uint32_t(uint64_t(work) * (xcd + 1) / kXcds) - first;
+        if (place < share) {
+            tile = bound[kind] + (first + place) / groups;
+            row_group = (first + place) % groups;
+            cols = kind == 0 ? uint32_t(mf::col_tiles) : (kind == 1 ? uint32_t(kNarrowCols) : uint32_t(kTinyCols));
+            return true;
+        }
+        place -= share;
     }
-    cols = cols_of_tile(header, tile);
-    return true;
+    return false;
+}
+
+// The grid for up to `tiles` tiles of `groups` row groups: the longest share has at most one
+// workgroup more per kind than an eighth of the work.
+dim3 xcd_grid(uint32_t groups, uint32_t tiles) {
+    return dim3(groups, tiles + (3 * kXcds + groups - 1) / groups);
 }
 
 // Accumulators: [matrix (gate 0/1, up 2/3)][column tile]; NC column tiles (by the tile's kind).
@@ -1857,7 +1870,7 @@ int ttl_matmul_mxfp4_selected(ttl_ctx *ctx, const ttl_mxfp4 *w, const float *bia
     m.plan = plan;
     m.out = out_dev;
     m.out_rows = x_rows;
-    matmul_kernel<3, true><<<dim3(w->rows / kMmRows, tiles), kMmWaves * 64, 0, ctx->stream>>>(m);
+    matmul_kernel<3, true><<<xcd_grid(w->rows / kMmRows, tiles), kMmWaves * 64, 0, ctx->stream>>>(m);
     TTL_LAUNCHED("matmul_kernel");
     return TTL_OK;
 }
@@ -1913,7 +1926,7 @@ int ttl_matmul_mxfp4_selected_mxfp8(ttl_ctx *ctx, const ttl_mxfp4 *w, const floa
     m.plan = plan;
     m.out = out_dev;
     m.out_rows = x_rows;
-    mx8_matmul_kernel<true><<<dim3(w->rows / kMmRows, tiles), kMmWaves * 64, 0, ctx->stream>>>(m);
+    mx8_matmul_kernel<true><<<xcd_grid(w->rows / kMmRows, tiles), kMmWaves * 64, 0, ctx->stream>>>(m);
     TTL_LAUNCHED("mx8_matmul_kernel");
     return TTL_OK;
 }
@@ -2049,7 +2062,7 @@ int moe_prefill_run(ttl_ctx *ctx, const ttl_moe_layer *layer, const void *x_dev,
     g.tiles_per_expert = L.gate->tiles;
     g.plan = plan;
     // one launch per GEMM over the wide tiles and the narrow and tiny ones (at most one per expert)
-    const dim3 gu_grid((L.expert_hidden + kGuRows - 1) / kGuRows, lay.tmax);
+    const dim3 gu_grid = xcd_grid((L.expert_hidden + kGuRows - 1) / kGuRows, lay.tmax);
     if ((stages & TTL_PREFILL_GATEUP) && scaled) {
         mx8_gateup_kernel<<<gu_grid, kGuWaves * 64, 0, ctx->stream>>>(g);
         TTL_LAUNCHED("mx8_gateup_kernel");
@@ -2082,14 +2095,14 @@ int moe_prefill_run(ttl_ctx *ctx, const ttl_moe_layer *layer, const void *x_dev,
     m.out = plan.down;
     m.out_rows = 0;
     if ((stages & TTL_PREFILL_DOWN) && scaled) {
-        mx8_matmul_kernel<false><<<dim3(L.hidden / kMmRows, lay.tmax), kMmWaves * 64, 0, ctx->stream>>>(m);
+        mx8_matmul_kernel<false><<<xcd_grid(L.hidden / kMmRows, lay.tmax), kMmWaves * 64, 0, ctx->stream>>>(m);
         TTL_LAUNCHED("mx8_matmul_kernel");
     } else if ((stages & TTL_PREFILL_DOWN) && f16h) {
         matmul_kernel<2, false, mf::f16x8, mf::kHiddenF16Shift>
-            <<<dim3(L.hidden / kMmRows, lay.tmax), kMmWaves * 64, 0, ctx->stream>>>(m);
+            <<<xcd_grid(L.hidden / kMmRows, lay.tmax), kMmWaves * 64, 0, ctx->stream>>>(m);
         TTL_LAUNCHED("matmul_kernel");
     } else if (stages & TTL_PREFILL_DOWN) {
-        matmul_kernel<kHiddenPlanes, false><<<dim3(L.hidden / kMmRows, lay.tmax), kMmWaves * 64, 0, ctx->stream>>>(m);
+        matmul_kernel<kHiddenPlanes, false><<<xcd_grid(L.hidden / kMmRows, lay.tmax), kMmWaves * 64, 0, ctx->stream>>>(m);
         TTL_LAUNCHED("matmul_kernel");
     }
     if (stages & TTL_PREFILL_COMBINE) {
