@@ -519,6 +519,40 @@ def test_moe_prefill_router_exact_path_in_a_batch(dev):
         device.free()
 
 
+# Logits that are the router's bias alone (a zero weight): ties within and across the
+# 64-position groups that a lane holds, both zeros, infinities and NaNs, also in the first
+# positions, against the reference's selection sort (model.cpp:296-309) spelled out.
+@pytest.mark.parametrize("experts,used", [(8, 8), (64, 4), (70, 16), (192, 5)])
+def test_moe_prefill_selection_ties_and_nan(dev, experts, used):
+    rs = np.random.RandomState(experts)
+    bias = rs.choice(np.array([0.0, -0.0, 1.0, 2.0, -3.0, np.nan, np.inf, -np.inf], np.float32), experts,
+                     p=[.2, .2, .2, .1, .1, .1, .05, .05])
+    host = HostLayer(experts, used, biases=True, seed=0x77000150, fill_experts=[])
+    host.router_w[:] = 0.0
+    device = DeviceLayer(dev, host)
+    count = 6
+    x = O.synth_normal(0x78000150, 0, count * N).reshape(count, N)
+    xb, out = dev.upload(x), dev.alloc(count * N * 4)
+    ib, wb = dev.alloc(count * used * 4), dev.alloc(count * used * 4)
+    try:
+        for shift in range(3):
+            b = np.roll(bias, shift * 3).astype(np.float32)
+            device.bufs[1].upload(b)
+            order = list(range(experts))
+            for i in range(used):
+                best = i
+                for j in range(i + 1, experts):
+                    if b[order[j]] > b[order[best]]:
+                        best = j
+                order[i], order[best] = order[best], order[i]
+            dev.moe_prefill(device.desc, xb, count, out, ib, wb)
+            assert np.array_equal(ib.download(np.int32).reshape(count, used), np.tile(order[:used], (count, 1)))
+    finally:
+        for buf in (xb, out, ib, wb):
+            buf.free()
+        device.free()
+
+
 def test_moe_prefill_zero_tokens_and_input_norm(dev, layer8):
     host, device = layer8
     out, xb = dev.alloc(256), dev.alloc(256)

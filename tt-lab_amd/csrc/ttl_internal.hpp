@@ -85,10 +85,11 @@ size_t moe_workspace_bytes();
 // for `device`, which must be current; once per device.
 int attention_scratch_init(int device);
 // Batched router of moe_batch (ttl_moe.hip): per-token exact rows in `scratch`
-// (router_scratch_bytes() each), indices/weights [count][used].
+// (router_scratch_bytes() each; the logits take at most 4 * 192 bytes of it, what follows is
+// free), indices/weights [count][used], shift (null or [count]) the f16-plane shifts of x's rows.
 size_t router_scratch_bytes();
 int launch_router_batch(ttl_ctx *ctx, const ttl_moe_layer &L, const float *x, uint32_t count, void *scratch,
-                        int32_t *indices, float *weights);
+                        int32_t *indices, float *weights, int32_t *shift);
 
 // The shift k of each of `rows` f32 rows (`cols` values each, a multiple of 4 and at most
 // 4096, rows `stride` floats apart, 16-byte aligned) for their two f16 planes: k of the

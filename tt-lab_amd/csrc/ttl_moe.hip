@@ -18,6 +18,7 @@
 //
 // route_workgroup() runs in one workgroup after the rows are known and publishes
 // indices, weights and logits; the gate/up kernel then reads the indices.
+#include "ttl_mfma.hpp"
 #include "ttl_moe_math.hpp"
 #include "ttl_mxfp4_tile.hpp"
 #include "ttl_stage.hpp"
@@ -837,22 +838,103 @@ __global__ __launch_bounds__(64 * W) void router_chain_batch_kernel(const float 
 }
 
 // The reference's selection sort and softmax (model.cpp:350-377) on a batch's exact
-// logits: one 64-thread workgroup per token.
+// logits: one 64-thread workgroup per token, lane l holding positions l, l + 64, l + 128 of
+// the sort's array in registers.  A step takes the largest non-NaN value at or after position
+// i (a wave maximum of order-preserving keys, -0 as +0), its first position (a ballot), and
+// swaps the two positions; it stays at i where i holds a NaN.  SHIFT: also the f16-plane
+// shift of the token's row of x (mf::row_shift of its largest finite magnitude), whose loads
+// land behind the logits'.  The replay in LDS with f64 shuffles that this took over from
+// took 6.3 us a launch at 40 tokens, and the shifts a launch of 4.9 us.
+template <bool SHIFT>
 __global__ __launch_bounds__(64) void router_select_logits_kernel(const float *__restrict__ logits,
                                                                   uint32_t experts, uint32_t k,
                                                                   int32_t *__restrict__ indices,
-                                                                  float *__restrict__ weights_out) {
-    __shared__ RouteLds lds;
+                                                                  float *__restrict__ weights_out,
+                                                                  const float *__restrict__ x,
+                                                                  int32_t *__restrict__ shift) {
+    __shared__ float selected[kMaxUsed], weights[kMaxUsed];
+    const uint32_t lane = threadIdx.x;
     const float *row = logits + size_t(blockIdx.x) * experts;
-    for (uint32_t c = threadIdx.x; c < experts; c += 64) {
-        lds.ref_logits[c] = row[c];
-        lds.order[c] = int32_t(c);
+    float value[kPerLane];
+    int32_t index[kPerLane];
+#pragma unroll
+    for (int j = 0; j < kPerLane; ++j) {
+        const uint32_t p = lane + 64 * j;
+        value[j] = row[p < experts ? p : 0u];
+        index[j] = int32_t(p);
+    }
+    constexpr int kRowQuads = kRouterCols / 4, kRowPer = (kRowQuads + 63) / 64;
+    float4 xr[SHIFT ? kRowPer : 1];
+    if constexpr (SHIFT) {
+        const float4 *xp = reinterpret_cast<const float4 *>(x + size_t(blockIdx.x) * kRouterCols);
+#pragma unroll
+        for (int j = 0; j < kRowPer; ++j) {
+            xr[j] = xp[min(lane + 64u * j, uint32_t(kRowQuads - 1))];
+        }
+    }
+    int32_t my_index = 0;  // lane r: rank r's expert
+    for (uint32_t i = 0; i < k; ++i) {
+        // position i (< 64) is lane i's first
+        const float start = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(value[0]), int(i)));
+        const int32_t start_index = __builtin_amdgcn_readlane(index[0], int(i));
+        uint32_t key[kPerLane], most = 0;
+#pragma unroll
+        for (int j = 0; j < kPerLane; ++j) {
+            const uint32_t p = lane + 64 * j;
+            key[j] = p >= i && p < experts && !isnan(value[j]) ? order_key32(value[j] + 0.0f) : 0u;
+            most = max(most, key[j]);
+        }
+        most = wave_max_u32(most);
+        float best_value = start;
+        int32_t best_index = start_index;
+        if (!isnan(start)) {  // (uniform, as the rest of the step)
+            bool found = false;
+#pragma unroll
+            for (int j = 0; j < kPerLane; ++j) {
+                const uint64_t at = __ballot(key[j] == most);
+                if (!found && at) {
+                    found = true;
+                    const int best = __builtin_ctzll(at);
+                    best_value = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(value[j]), best));
+                    best_index = __builtin_amdgcn_readlane(index[j], best);
+                    if (lane == uint32_t(best)) {
+                        value[j] = start;
+                        index[j] = start_index;
+                    }
+                }
+            }
+            if (lane == i) {
+                value[0] = best_value;
+                index[0] = best_index;
+            }
+        }
+        if (lane == i) {
+            my_index = best_index;
+            selected[i] = best_value;
+        }
     }
     __syncthreads();
-    replay_selection(experts, k, nullptr, lds, false);
-    if (threadIdx.x < k) {
-        indices[size_t(blockIdx.x) * k + threadIdx.x] = lds.indices[threadIdx.x];
-        weights_out[size_t(blockIdx.x) * k + threadIdx.x] = lds.weights[threadIdx.x];
+    if (lane == 0) {
+        softmax_selected(selected, k, weights);
+    }
+    if constexpr (SHIFT) {
+        float m = 0.0f;
+#pragma unroll
+        for (int j = 0; j < kRowPer; ++j) {
+            m = mf::finite_max(mf::finite_max(mf::finite_max(mf::finite_max(m, xr[j].x), xr[j].y), xr[j].z), xr[j].w);
+        }
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) {
+            m = __builtin_fmaxf(m, __shfl_xor(m, d));
+        }
+        if (lane == 0) {
+            shift[blockIdx.x] = mf::row_shift(m);
+        }
+    }
+    __syncthreads();
+    if (lane < k) {
+        indices[size_t(blockIdx.x) * k + lane] = my_index;
+        weights_out[size_t(blockIdx.x) * k + lane] = weights[lane];
     }
 }
 
@@ -1452,8 +1534,9 @@ size_t router_scratch_bytes() {
 // logits in the reference's order go to the scratch (count * experts floats), its
 // indices and weights to indices/weights + t * used.  The logits are exact, so no
 // certificate and no fallback: a batch costs the same whatever its ties.
+// shift (int32 [count], or null) receives the f16-plane shifts of the rows of x.
 int launch_router_batch(ttl_ctx *ctx, const ttl_moe_layer &L, const float *x, uint32_t count, void *scratch,
-                        int32_t *indices, float *weights) {
+                        int32_t *indices, float *weights, int32_t *shift) {
     const int rc = check_router(L.router_weight, L.router_bias, L.experts, L.hidden, x, L.used);
     if (rc != TTL_OK) {
         return rc;
@@ -1462,13 +1545,19 @@ int launch_router_batch(ttl_ctx *ctx, const ttl_moe_layer &L, const float *x, ui
     TTL_REQUIRE(!L.input_norm, TTL_ERR_INVALID, "moe_batch router: x is the normalized router input");
     // the logits in the reference's order (the scratch holds count * experts floats),
     // then the selection
-    static_assert(sizeof(RouterScratch) >= 4 * kMaxExperts, "a token's scratch holds its logits");
+    static_assert(sizeof(RouterScratch) >= 4 * kMaxExperts + 4, "a token's scratch holds its logits and its shift");
     float *logits = static_cast<float *>(scratch);
     constexpr int W = 4;
     router_chain_batch_kernel<W>
         <<<dim3((count + kRcTokens - 1) / kRcTokens, (L.experts + W - 1) / W), 64 * W, 0, ctx->stream>>>(
             L.router_weight, L.router_bias, x, L.hidden, count, L.experts, logits);
-    router_select_logits_kernel<<<count, 64, 0, ctx->stream>>>(logits, L.experts, L.used, indices, weights);
+    if (shift) {
+        router_select_logits_kernel<true>
+            <<<count, 64, 0, ctx->stream>>>(logits, L.experts, L.used, indices, weights, x, shift);
+    } else {
+        router_select_logits_kernel<false>
+            <<<count, 64, 0, ctx->stream>>>(logits, L.experts, L.used, indices, weights, nullptr, nullptr);
+    }
     TTL_LAUNCHED("moe_batch router kernels");
     return TTL_OK;
 }

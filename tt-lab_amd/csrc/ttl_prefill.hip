@@ -2211,14 +2211,20 @@ int ttl_moe_prefill_fused(ttl_ctx *ctx, const ttl_moe_layer *layer, const float 
     float *weights = reinterpret_cast<float *>(w);
     w += align256(4ull * count * layer->used);
     const size_t rest = workspace_bytes - size_t(w - static_cast<uint8_t *>(workspace_dev));
+    // the f16-plane shifts, where the GEMMs use them and the caller has none, come with the
+    // selection, into the router's scratch behind the logits
+    int32_t *shift = nullptr;
+    if (!x_shift_dev && layer->gate->f16_exact() && layer->up->f16_exact()) {
+        shift = static_cast<int32_t *>(scratch) + size_t(count) * layer->experts;
+    }
     int rc = ttl::launch_router_batch(ctx, *layer, x_dev, count, scratch, indices_dev ? indices_dev : indices,
-                                      weights_dev ? weights_dev : weights);
+                                      weights_dev ? weights_dev : weights, shift);
     if (rc != TTL_OK) {
         return rc;
     }
     return moe_prefill_run(ctx, layer, x_dev, TTL_DTYPE_F32, count, indices_dev ? indices_dev : indices,
-                           weights_dev ? weights_dev : weights, out_dev, w, rest, TTL_PREFILL_ALL, x_shift_dev,
-                           residual_dev);
+                           weights_dev ? weights_dev : weights, out_dev, w, rest, TTL_PREFILL_ALL,
+                           shift ? shift : x_shift_dev, residual_dev);
 }
 
 int ttl_moe_prefill(ttl_ctx *ctx, const ttl_moe_layer *layer, const float *x_dev, uint32_t count, float *out_dev,
