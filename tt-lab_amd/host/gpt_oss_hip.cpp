@@ -434,7 +434,9 @@ const float *HipGptOssModel::forward(int32_t token, size_t position) {
 // tokens already in prefill_tokens_, at positions first .. first + count - 1.  The
 // per-token results do not depend on how a prompt is cut into passes: each pass's
 // attention reads the earlier positions' keys and values from the caches.
-int HipGptOssModel::enqueue_prefill_chunk(size_t first, size_t count) {
+// `last`: the prompt ends here, and the pass ends with its logits (172 us of unembedding
+// that the passes before it need not read).
+int HipGptOssModel::enqueue_prefill_chunk(size_t first, size_t count, bool last) {
     const size_t L = spec_.layers, B = prefill_batch_;
     const uint32_t n = uint32_t(count);
     int status = ttl_embedding_q8_0_batch(ctx_, embedding_, spec_.vocab, prefill_tokens_, n, x_seq_);
@@ -473,7 +475,7 @@ int HipGptOssModel::enqueue_prefill_chunk(size_t first, size_t count) {
                                            nullptr, moe_workspace_, moe_workspace_bytes_);
         }
     }
-    if (status == TTL_OK) {
+    if (status == TTL_OK && last) {
         // model.cpp:555-559: the logits of the last token
         ttl_stage_input f{};
         f.base = x_seq_ + (L * B + count - 1) * kHidden;
@@ -512,7 +514,7 @@ const float *HipGptOssModel::prefill(const int32_t *tokens, size_t count) {
     for (size_t first = 0; first < count; first += prefill_batch_) {
         const size_t n = std::min(prefill_batch_, count - first);
         check(ttl_memcpy_h2d(ctx_, prefill_tokens_, tokens + first, sizeof(int32_t) * n), "ttl_memcpy_h2d");
-        check(enqueue_prefill_chunk(first, n), "prefill");
+        check(enqueue_prefill_chunk(first, n, first + n == count), "prefill");
     }
     check(ttl_memcpy_d2h(ctx_, host_logits_, logits_, sizeof(float) * spec_.vocab), "ttl_memcpy_d2h");
     return host_logits_;

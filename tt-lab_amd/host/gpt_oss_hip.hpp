@@ -194,7 +194,7 @@ class HipGptOssModel {
     void finish_construction();
     int enqueue_step();
     ttl_stage_input layer_input(size_t layer, const float *norm_weight) const;
-    int enqueue_prefill_chunk(size_t first, size_t count);
+    int enqueue_prefill_chunk(size_t first, size_t count, bool last);
     void record_step();
     void run_step();
     void set_position(int32_t token, size_t position);
