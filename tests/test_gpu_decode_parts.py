@@ -3,6 +3,8 @@ Q8_0 matvec (with the fused combine / RMSNorm staging), the fused Q/K/V projecti
 with RoPE and the KV-cache store, attention with sinks, the bf16 unembedding,
 greedy argmax and the embedding lookup.  Tolerance: relative L2 <= 1e-5; argmax,
 layout round trips and the staging's combine are bit-exact."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -289,6 +291,50 @@ def test_attention_prefill_matches_oracle_per_token(dev, layer_index, first, tok
     print(f"attention prefill layer {layer_index} positions {first}..{last}: worst rel_l2 {worst:.2e}")
     assert worst <= TOL
     for b in (qb, kb, vb, sb, out):
+        b.free()
+
+
+# The batched bias + RoPE + KV store, token by token in f32 with every product rounded, so
+# bit for bit.  A workgroup takes 256 of the 640 half tiles of each token: token counts whose
+# last workgroup is full and partly empty; one array four bytes off its 16-byte alignment
+# takes the kernel that loads and stores single floats.
+@pytest.mark.parametrize("tokens,first,off", [(1, 0, None), (2, 5, None), (7, 3, None), (1, 0, "qkv"), (3, 2, "bias"),
+                                              (3, 0, "rope"), (5, 1, "q"), (2, 9, "k"), (2, 4, "v")])
+def test_qkv_rope_store_batch(dev, tokens, first, off):
+    capacity = first + tokens + 1
+    rows = np.empty(5120, np.int32)
+    lib = ttlab_amd.load_library()
+    lib.ttl_qkv_row_source(rows.ctypes.data)
+    qkv = O.synth_normal(81, tokens, tokens * 5120).reshape(tokens, 5120)
+    bias = O.synth_normal(82, 0, 5120, sigma=0.3)
+    angle = np.random.RandomState(first).rand(capacity, 32) * 6.0
+    rope = np.stack([np.cos(angle), np.sin(angle)], -1).astype(np.float32)
+    arrays = {"qkv": qkv, "bias": bias, "rope": rope, "q": np.full(tokens * 4096 + 4, 7.0, np.float32),
+              "k": np.full(capacity * 512, 7.0, np.float32), "v": np.full(capacity * 512, 7.0, np.float32)}
+    bufs, at = {}, {}
+    for name, a in arrays.items():
+        pad = 1 if name == off else 0
+        bufs[name] = dev.upload(np.concatenate([np.zeros(pad, np.float32), a.ravel().astype(np.float32)]))
+        at[name] = C.c_void_p(bufs[name].ptr + 4 * pad)
+    ttlab_amd._check(lib.ttl_qkv_rope_store(C.c_void_p(dev.ctx), at["qkv"], C.c_uint32(tokens), C.c_uint32(first),
+                                            at["bias"], at["rope"], C.c_uint32(capacity), at["q"], at["k"], at["v"]),
+                     "ttl_qkv_rope_store")
+    got = {n: bufs[n].download(np.float32)[1 if n == off else 0:] for n in ("q", "k", "v")}
+    y = np.empty((tokens, 5120), np.float32)
+    y[:, rows] = bias[rows] + qkv
+    cs, sn = rope[first:first + tokens, None, :, 0], rope[first:first + tokens, None, :, 1]
+
+    def rotate(h):
+        lo, hi = h[..., :32], h[..., 32:]
+        return np.concatenate([lo * cs - hi * sn, lo * sn + hi * cs], -1)
+
+    want = {n: arrays[n].copy() for n in ("q", "k", "v")}
+    want["q"][:tokens * 4096] = rotate(y[:, :4096].reshape(tokens, 64, 64)).ravel()
+    want["k"][first * 512:(first + tokens) * 512] = rotate(y[:, 4096:4608].reshape(tokens, 8, 64)).ravel()
+    want["v"][first * 512:(first + tokens) * 512] = y[:, 4608:].ravel()
+    for n in want:
+        assert np.array_equal(got[n].view(np.uint32), want[n].view(np.uint32)), n
+    for b in bufs.values():
         b.free()
 
 
