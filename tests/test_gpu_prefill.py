@@ -519,6 +519,41 @@ def test_moe_prefill_router_exact_path_in_a_batch(dev):
         device.free()
 
 
+# Router rows that differ in their last bits only: a token's logits lie a few ulps apart, in
+# the order that the reference's own sequence of rounded products and sums gives them, so any
+# other order of the sums shows in the indices.  Batches and expert counts at and around the
+# 4 tokens x 16 experts of a workgroup.
+@pytest.mark.parametrize("count", [1, 3, 4, 5, 9])
+@pytest.mark.parametrize("experts,used", [(8, 8), (16, 16), (17, 16), (33, 16)])
+def test_moe_prefill_router_order_of_sums(dev, experts, used, count):
+    host = HostLayer(experts, used, biases=True, seed=0x77000160, fill_experts=[])
+    rs = np.random.RandomState(experts + count)
+    row = O.synth_normal(0x78000160, 0, N, sigma=0.02)
+    host.router_w = np.ascontiguousarray(
+        (row[None, :] * (1.0 + 1e-7 * rs.randn(experts, N))).astype(np.float32).ravel())
+    device = DeviceLayer(dev, host)
+    x = O.synth_normal(0x78000160, 1, count * N).reshape(count, N)
+    xb, out, bias = dev.upload(x), dev.alloc(count * N * 4), np.full(experts, 0.125, np.float32)
+    ib, wb = dev.alloc(count * used * 4), dev.alloc(count * used * 4)
+    try:
+        device.bufs[1].upload(bias)
+        dev.moe_prefill(device.desc, xb, count, out, ib, wb)
+        got = ib.download(np.int32).reshape(count, used)
+        w = host.router_w.reshape(experts, N)
+        distinct = 0
+        for p in range(count):
+            steps = np.concatenate([bias[:, None], w * x[p][None, :]], axis=1)
+            logits = np.add.accumulate(steps, axis=1, dtype=np.float32)[:, -1]  # in column order
+            idx, _ = O.router_topk(np.ascontiguousarray(logits), used)
+            assert list(got[p]) == list(idx), p
+            distinct += np.unique(logits).size
+        assert distinct > 2 * count  # (the order does say something)
+    finally:
+        for buf in (xb, out, ib, wb):
+            buf.free()
+        device.free()
+
+
 # Logits that are the router's bias alone (a zero weight): ties within and across the
 # 64-position groups that a lane holds, both zeros, infinities and NaNs, also in the first
 # positions, against the reference's selection sort (model.cpp:296-309) spelled out.
