@@ -380,6 +380,55 @@ def test_attention_prefill_wide_values(dev, layer_index, kind):
     check_attention_prefill(dev, q, k, v, sinks, layer_index, first, tokens, capacity)
 
 
+# A sink decides most of the denominator here and lies where f32 holds units of log 2 worst
+# (129 to 133, its product with log2 e close to half way between two values), while the one
+# score's product is close to a value.  The sink's weight alone would be off by 4.7e-6 if it
+# were rounded; what is left is a few f32 roundings of the result (2^-24 each): 1e-6.
+def test_attention_prefill_sink_keeps_its_bits(dev):
+    rs = np.random.RandomState(5)
+    log2e = 1.4426950408889634
+
+    def off_grid(x):  # distance of x log2 e from f32, in its last places
+        v = x.astype(np.float64) * log2e
+        return np.abs(v - v.astype(np.float32)) / np.spacing(v.astype(np.float32)).astype(np.float64)
+
+    scores, sinks = [(lo + (hi - lo) * rs.rand(20000)).astype(np.float32) for lo, hi in ((86.0, 88.5), (89.5, 92.0))]
+    scores = scores[np.argsort(off_grid(scores))[:64]]
+    sinks = sinks[np.argsort(-off_grid(sinks))[:64]]
+    assert off_grid(scores).max() < 0.02 and off_grid(sinks).min() > 0.45
+    q, k, v = np.zeros((64, 64), np.float32), np.zeros((8, 64), np.float32), O.synth_normal(65, 0, 512)
+    q[:, 0], k[:, 0] = scores * 8.0, 1.0
+    bufs = [dev.upload(a) for a in (q.ravel(), k.ravel(), v, sinks)]
+    out = dev.alloc(4096 * 4)
+    dev.attention_prefill(*bufs, 0, 1, 1, 1, out)
+    got = out.download(np.float32).reshape(64, 64)
+    e = np.exp(scores.astype(np.float64) - sinks.astype(np.float64))
+    want = (e / (e + 1.0))[:, None] * np.repeat(v.reshape(8, 64), 8, axis=0).astype(np.float64)
+    err = np.linalg.norm(got - want, axis=1) / np.linalg.norm(want, axis=1)
+    assert err.max() <= 1e-6, err.max()
+    for b in bufs + [out]:
+        b.free()
+
+
+# Sinks whose product with log2 e is past the largest f32, both signs, infinite and NaN, next
+# to ordinary ones, on the bf16 planes and (K infinite) on f32 MFMA.  (60: exp(score - 60) is
+# still a normal f32 in the oracle.)
+@pytest.mark.parametrize("layer_index", [0, 1])
+@pytest.mark.parametrize("k_inf", [False, True])
+def test_attention_prefill_extreme_sinks(dev, layer_index, k_inf):
+    first, tokens = 150, 20
+    capacity = first + tokens
+    q = O.synth_normal(75, 0, tokens * 4096, sigma=2.0)
+    k = O.synth_normal(76, 0, capacity * 512, sigma=2.0)
+    v = O.synth_normal(77, 0, capacity * 512)
+    sinks = O.synth_normal(78, 0, 64, sigma=2.0)
+    big = np.finfo(np.float32).max
+    sinks[:64:9] = [2.4e38, -2.4e38, big, -big, np.inf, -np.inf, np.nan, 60.0]
+    if k_inf:
+        k.reshape(capacity, 8, 64)[140, 3, 5] = np.inf
+    check_attention_prefill(dev, q, k, v, sinks, layer_index, first, tokens, capacity)
+
+
 def check_attention_prefill(dev, q, k, v, sinks, layer_index, first, tokens, capacity):
     bufs = [dev.upload(a) for a in (q, k, v, sinks)]
     out = dev.alloc(tokens * 4096 * 4)

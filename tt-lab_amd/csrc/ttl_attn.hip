@@ -348,14 +348,13 @@ __global__ __launch_bounds__(kWinThreads) void attn_window_kernel(const float *_
 // group times 16 tokens are 128 queries, in tiles of 16, two tiles per wave of a group of
 // four waves.  Two such groups share the workgroup and take the chunks of 64 positions in
 // turn (group 0 the first, third, ..., group 1 the others), each with an online softmax
-// of its own; group 0 merges the two at the end.  Per chunk and query tile:
+// of its own.  Per chunk and query tile:
 //  - S^T (positions x queries) = K Q^T, then an online softmax per query (a column of S^T:
-//    the lane's 4 rows of each position tile and the 4 lanes of its column).  m starts at
-//    the sink and l (group 0) at exp(sink - sink) = 1, so the sink takes part in the max
-//    and the denominator (model.cpp:270-281); per chunk m' = max(m, scores), and l and O
-//    are rescaled by exp(m - m');
+//    the lane's 4 rows of each position tile and the 4 lanes of its column): m' = max(m,
+//    scores), and l and O are rescaled by exp(m - m');
 //  - O^T (dims x queries) += V^T P^T.
-// The output is O / l.
+// At the end group 0 merges the two states and the sink, which takes part in the maximum
+// and the denominator (model.cpp:270-281).  The output is O / l.
 //
 // v_mfma_f32_16x16x32_bf16 (D = A B + C): lane (n, g) = (l % 16, l / 16) holds 8 bf16 of
 // A row n and of B column n for 8 of the 32 K indices, the same for A and B, and receives
@@ -444,7 +443,16 @@ constexpr int kPfKMax = 60, kPfVMax = 100;  // and 2^60 for the queries
 // Scores and their maxima are kept in units of log 2 (times log2 e), so a probability is
 // one v_exp_f32 (1 ulp); the factor goes into the queries, carried past f32.
 constexpr float kLog2e = 0x1.715476p+0f, kLog2eLo = 0x1.4ae0cp-26f;  // log2 e = their sum
-constexpr float kPfMasked = -3.0e38f;  // a masked score: exp2 of its distance to any maximum is zero
+
+// A sink in units of log 2, as a value and what f32 rounds off it (of sinks small enough that
+// it says something).  Scores are an f32 dot product / 8 and stay finite in these units; a
+// sink of 2^127 may not, and the largest f32 outweighs every finite score as it does.
+__device__ inline float sink_log2(float sink, float &lo) {
+#pragma clang fp contract(off)
+    const float hi = sink * kLog2e;
+    lo = fabsf(sink) < 0x1p14f ? fmaf(sink, kLog2eLo, fmaf(sink, kLog2e, -hi)) : 0.0f;
+    return isinf(hi) && !isinf(sink) ? copysignf(0x1.fffffep+127f, sink) : hi;
+}
 
 // The online softmax state of a wave's queries.
 struct PfState {
@@ -453,14 +461,14 @@ struct PfState {
 };
 
 // The running maximum and rescaling of one query tile for a chunk whose largest score of
-// the lane is cmax.  (A sink of -infinity and a chunk masked as a whole: the maximum is
-// kPfMasked or -infinity, and the first real score's rescaling takes what was summed to
-// zero.)
+// the lane is cmax; returns what to subtract from the chunk's scores: the maximum, or zero
+// while every score was masked (-infinity, whose exp2 is zero).
 __device__ __attribute__((always_inline)) inline float pf_rescale(PfState &st, int qi, float cmax) {
     cmax = fmaxf(cmax, __shfl_xor(cmax, 16));
     cmax = fmaxf(cmax, __shfl_xor(cmax, 32));
     const float m2 = fmaxf(st.m[qi], cmax);
-    const float scale = m2 == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(st.m[qi] - m2);
+    const float base = m2 == -INFINITY ? 0.0f : m2;
+    const float scale = __builtin_amdgcn_exp2f(st.m[qi] - base);
     st.l[qi] *= scale;
     st.m[qi] = m2;
 #pragma unroll
@@ -470,7 +478,7 @@ __device__ __attribute__((always_inline)) inline float pf_rescale(PfState &st, i
             st.o[qi][mt][i] *= scale;
         }
     }
-    return m2;
+    return base;
 }
 
 // One chunk on f32 MFMA, operands straight from global memory: K step (s, j) of the scores
@@ -598,6 +606,7 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2)))
     // this lane's query (column n) of each of the wave's tiles, as B fragments of K step s
     uint32_t qp[kPfTiles][2][kPfPlanes][4];
     uint32_t qpos[kPfTiles], qfirst[kPfTiles], qrow[kPfTiles];
+    float sink[kPfTiles];
     bool live[kPfTiles];
     PfState st;
     uint32_t bad_query = 0;
@@ -626,8 +635,9 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2)))
                 }
             }
         }
-        st.m[qi] = sinks[head] * kLog2e;
-        st.l[qi] = g == 0 && grp == 0 ? 1.0f : 0.0f;  // the sink's exp(sink - m), counted once per column
+        sink[qi] = sinks[head];
+        st.m[qi] = -INFINITY;
+        st.l[qi] = 0.0f;
 #pragma unroll
         for (int mt = 0; mt < 4; ++mt) {
             st.o[qi][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -757,7 +767,7 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2)))
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         const uint32_t at = c0 + 16 * p + 4 * g + i;
-                        sc[qi][p][i] = at >= qfirst[qi] && at <= qpos[qi] ? sc[qi][p][i] : kPfMasked;
+                        sc[qi][p][i] = at >= qfirst[qi] && at <= qpos[qi] ? sc[qi][p][i] : -INFINITY;
                     }
                 }
             }
@@ -850,11 +860,14 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2)))
     for (int qi = 0; qi < kPfTiles; ++qi) {
         const float *d = hand + qi * kState * 64;
         const float m1 = d[0];
-        const float m = fmaxf(st.m[qi], m1);
+        float sink_lo;
+        const float sink_hi = sink_log2(sink[qi], sink_lo);
+        const float m = fmaxf(fmaxf(st.m[qi], m1), sink_hi);
         const float w0 = __builtin_amdgcn_exp2f(st.m[qi] - m), w1 = __builtin_amdgcn_exp2f(m1 - m);
         float den = st.l[qi] * w0 + d[64] * w1;
         den += __shfl_xor(den, 16);
         den += __shfl_xor(den, 32);
+        den += __builtin_amdgcn_exp2f((sink_hi - m) + sink_lo);
         if (live[qi]) {
             float *dst = out + size_t(qrow[qi]) * kHead;
 #pragma unroll
