@@ -410,6 +410,22 @@ def test_attention_prefill_sink_keeps_its_bits(dev):
         b.free()
 
 
+# A V that is not finite at a position that a query does not see, of the same block of 16
+# tokens (later ones) or one that the window has passed (earlier ones): no output holds it
+# but those that the oracle has it in.
+@pytest.mark.parametrize("layer_index", [0, 1])
+@pytest.mark.parametrize("position", [71, 80, 200, 209, 230, 239])
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+def test_attention_prefill_v_outside_the_span(dev, layer_index, position, value):
+    first, tokens = 200, 40
+    capacity = first + tokens
+    q = O.synth_normal(85, 0, tokens * 4096, sigma=2.0)
+    k = O.synth_normal(86, 0, capacity * 512, sigma=2.0)
+    v = O.synth_normal(87, 0, capacity * 512)
+    v.reshape(capacity, 8, 64)[position, 6, 17] = value
+    check_attention_prefill(dev, q, k, v, O.synth_normal(88, 0, 64), layer_index, first, tokens, capacity)
+
+
 # Sinks whose product with log2 e is past the largest f32, both signs, infinite and NaN, next
 # to ordinary ones, on the bf16 planes and (K infinite) on f32 MFMA.  (60: exp(score - 60) is
 # still a normal f32 in the oracle.)

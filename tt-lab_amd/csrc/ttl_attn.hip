@@ -483,7 +483,9 @@ __device__ __attribute__((always_inline)) inline float pf_rescale(PfState &st, i
 
 // One chunk on f32 MFMA, operands straight from global memory: K step (s, j) of the scores
 // covers dims 16s + 4k + j for lane group k; K step j of position tile p of the second
-// product takes positions 16p + 4k + j.
+// product takes positions 16p + 4k + j.  A query's probabilities are zero outside its span,
+// but zero times an infinite V is not: the second product runs once for each of the tile's
+// two tokens, with that token's span of V rows, and a query keeps its own token's sums.
 struct PfQueries {
     uint32_t row[kPfTiles], first[kPfTiles], pos[kPfTiles];
 };
@@ -530,16 +532,24 @@ __device__ __attribute__((noinline)) void attn_chunk_f32(const float *q, const f
                 st.l[qi] += sc[p][i];
             }
         }
+        static_assert(kGroup == 8, "a tile's queries are two tokens' 8 heads");
+        // (the tile's token u: query columns 8u..8u+7)
+        const uint32_t first0 = __shfl(qs.first[qi], 0), pos0 = __shfl(qs.pos[qi], 0);
+        const uint32_t first1 = __shfl(qs.first[qi], 8), pos1 = __shfl(qs.pos[qi], 8);
+#pragma unroll 1
+        for (int mt = 0; mt < 4; ++mt) {
+            f32x4 o0 = st.o[qi][mt], o1 = o0;
 #pragma unroll
-        for (int p = 0; p < 4; ++p) {
+            for (int p = 0; p < 4; ++p) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const size_t row = (size_t(min(c0 + 16 * p + 4 * g + j, hi)) * kKvHeads + kvh) * kHead;
-#pragma unroll
-                for (int mt = 0; mt < 4; ++mt) {
-                    st.o[qi][mt] = mfma_f32(v_cache[row + 16 * mt + n], sc[p][j], st.o[qi][mt]);
+                for (int j = 0; j < 4; ++j) {
+                    const uint32_t at = c0 + 16 * p + 4 * g + j;
+                    const float v = v_cache[(size_t(min(at, hi)) * kKvHeads + kvh) * kHead + 16 * mt + n];
+                    o0 = mfma_f32(at >= first0 && at <= pos0 ? v : 0.0f, sc[p][j], o0);
+                    o1 = mfma_f32(at >= first1 && at <= pos1 ? v : 0.0f, sc[p][j], o1);
                 }
             }
+            st.o[qi][mt] = n < 8 ? o0 : o1;
         }
     }
 }
