@@ -382,8 +382,8 @@ def test_attention_prefill_wide_values(dev, layer_index, kind):
 
 # A sink decides most of the denominator here and lies where f32 holds units of log 2 worst
 # (129 to 133, its product with log2 e close to half way between two values), while the one
-# score's product is close to a value.  The sink's weight alone would be off by 4.7e-6 if it
-# were rounded; what is left is a few f32 roundings of the result (2^-24 each): 1e-6.
+# score's product is close to a value.  The result is off by 5.3e-6 if the sink is rounded;
+# what is left otherwise is a few f32 roundings of the result (2^-24 each): 1e-6.
 def test_attention_prefill_sink_keeps_its_bits(dev):
     rs = np.random.RandomState(5)
     log2e = 1.4426950408889634
@@ -408,6 +408,32 @@ def test_attention_prefill_sink_keeps_its_bits(dev):
     assert err.max() <= 1e-6, err.max()
     for b in bufs + [out]:
         b.free()
+
+
+# V below what three bf16 planes hold (2^-100): every one; one dim's; those of a few
+# positions of one parity, and of one position alone among zeros.  Within the usual bar of
+# the oracle, whose products of 2^-119 and a probability keep at least 17 bits.
+@pytest.mark.parametrize("layer_index", [0, 1])
+@pytest.mark.parametrize("kind", ["all", "dim", "parity", "one"])
+def test_attention_prefill_small_values(dev, layer_index, kind):
+    first, tokens = 90, 40
+    capacity = first + tokens
+    q = O.synth_normal(81, 0, tokens * 4096)
+    k = O.synth_normal(82, 0, capacity * 512)
+    v = O.synth_normal(83, 0, capacity * 512)
+    v3 = v.reshape(capacity, 8, 64)
+    small = v3 * np.float32(2.0**-119)
+    if kind == "all":
+        v3[:] = small
+    elif kind == "dim":
+        v3[:, 5, 11] = small[:, 5, 11]
+    else:
+        at = slice(65, 80, 2) if kind == "parity" else 99
+        v3[:, 5] = 0.0
+        v3[at, 5] = small[at, 5]
+    got, ref = check_attention_prefill(dev, q, k, v, O.synth_normal(84, 0, 64), layer_index, first, tokens, capacity)
+    d = got[:, 40:48, 11].astype(np.float64) - ref[:, 40:48, 11]  # the dim by itself
+    assert np.linalg.norm(d) <= TOL * np.linalg.norm(ref[:, 40:48, 11].astype(np.float64))
 
 
 # A V that is not finite at a position that a query does not see, of the same block of 16
@@ -450,7 +476,7 @@ def check_attention_prefill(dev, q, k, v, sinks, layer_index, first, tokens, cap
     out = dev.alloc(tokens * 4096 * 4)
     dev.attention_prefill(*bufs, first, tokens, capacity, layer_index, out)
     got = out.download(np.float32).reshape(tokens, 64, 64)
-    ref = np.empty(4096, np.float32)
+    ref, refs = np.empty(4096, np.float32), np.empty_like(got)
     scores = np.empty(capacity, np.float32)
     for t in range(tokens):
         O.lib.orc_attention(np.ascontiguousarray(q[t * 4096:(t + 1) * 4096]), k, v, sinks, layer_index, first + t,
@@ -463,8 +489,10 @@ def check_attention_prefill(dev, q, k, v, sinks, layer_index, first, tokens, cap
             f = fine[h]
             err = np.linalg.norm((got[t, h][f] - r[h][f]).astype(np.float64))
             assert err <= TOL * np.linalg.norm(r[h][f].astype(np.float64)), (t, h)
+        refs[t] = r
     for b in bufs + [out]:
         b.free()
+    return got, refs
 
 
 def test_attention_prefill_rejects_bad_shapes(dev):

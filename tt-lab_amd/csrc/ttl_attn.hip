@@ -364,13 +364,17 @@ __global__ __launch_bounds__(kWinThreads) void attn_window_kernel(const float *_
 // rows of the lane's own S^T tiles, so the probabilities never leave their registers; V is
 // staged transposed, with the positions of a dim in that order.
 //
-// Numerics: x = x0 + x1 + x2, each plane the remainder rounded to bf16, holds every f32 to
-// its last bit or 2^-25 of it; the products x0 y0, x0 y1, x1 y0, x1 y1, x0 y2, x2 y0 are
+// Numerics: x = x0 + x1 + x2, each plane the remainder rounded to bf16, holds every f32 of
+// 2^-100 or more to its last bit or 2^-25 of it; the products x0 y0, x0 y1, x1 y0, x1 y1, x0 y2, x2 y0 are
 // exact in f32 and the three left out are at most 2^-24 of |x y|, as much as f32 rounds
 // the product itself.  Relative error against 64 bits, 512 tokens at 1536 (a sliding and a
 // full layer): 3.9e-7 on f32 MFMA, 2.4e-7 this way.  The planes assume magnitudes whose
 // sums stay finite: a chunk with a K of 2^60 or more, a V of 2^100 or more, an infinity or
-// a NaN, and every chunk of a block with such a query, takes f32 MFMA (attn_chunk_f32).
+// a NaN, and every chunk of a block with such a query, takes f32 MFMA (attn_chunk_f32).  So
+// does a chunk with V that the planes run out of exponent for: eight V of one dim and parity
+// of position below 2^-100 and not all zero.  (Of a smaller value among larger ones they
+// hold 2^-134, of a probability the same: 2^-34 of the largest.  Small queries and keys
+// need no more: their scores are next to zero.)
 //
 // What bounds it: on v_mfma_f32_16x16x4_f32 a chunk's two products of a wave take 256
 // instructions of 32 cycles; six bf16 products take 192 of 16, and the second group puts a
@@ -427,7 +431,7 @@ __device__ __attribute__((always_inline)) inline void split3_scaled(float a, flo
 }
 
 // The larger magnitudes of two packed pairs of bf16 (as bit patterns, so infinities and
-// NaNs are the largest), and whether one of a pair is 2^E or more.
+// NaNs are the largest), and whether one of a pair, or each, is 2^E or more.
 __device__ inline uint32_t pair_max(uint32_t acc, uint32_t w) {
     typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
     return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, acc),
@@ -438,7 +442,13 @@ __device__ inline bool at_least(uint32_t pair) {
     constexpr uint32_t bits = uint32_t(E + 127) << 7;
     return (pair & 0xffffu) >= bits || (pair >> 16) >= bits;
 }
+template <int E>
+__device__ inline bool both_at_least(uint32_t pair) {
+    constexpr uint32_t bits = uint32_t(E + 127) << 7;
+    return (pair & 0xffffu) >= bits && (pair >> 16) >= bits;
+}
 constexpr int kPfKMax = 60, kPfVMax = 100;  // and 2^60 for the queries
+constexpr int kPfVMin = -100;
 
 // Scores and their maxima are kept in units of log 2 (times log2 e), so a probability is
 // one v_exp_f32 (1 ulp); the factor goes into the queries, carried past f32.
@@ -712,7 +722,14 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2)))
                     *reinterpret_cast<u32x2 *>(vd + p * kPfPlane + k * 128) = u32x2{w0[p], w1[p]};
                 }
             }
-            if (at_least<kPfKMax>(bad_k) || at_least<kPfVMax>(bad_v)) {
+            bool off = at_least<kPfKMax>(bad_k) || at_least<kPfVMax>(bad_v);
+            if (!both_at_least<kPfVMin>(bad_v)) {  // the thread's V of a parity all small: zeros, or not?
+#pragma unroll
+                for (int k = 0; k < 16; ++k) {
+                    off |= vr[k] != 0.0f && fabsf(vr[k]) < __builtin_ldexpf(1.0f, kPfVMin);
+                }
+            }
+            if (off) {
                 odd[grp][round % 2] = 1;
             }
         }
