@@ -526,6 +526,19 @@ def test_moe_prefill_router_exact_path_in_a_batch(dev):
 @pytest.mark.parametrize("count", [1, 3, 4, 5, 9])
 @pytest.mark.parametrize("experts,used", [(8, 8), (16, 16), (17, 16), (33, 16)])
 def test_moe_prefill_router_order_of_sums(dev, experts, used, count):
+    check_router_order_of_sums(dev, experts, used, count)
+
+
+# The same around the 512 workgroups of 4 x 16 (on 256 CUs) past which a launch has a lane per
+# logit, 64 tokens x 4 experts a workgroup: 510 and 513 of them, 504 and 513, 512 and 513; the
+# last group of tokens with 1, 33 or 41, of experts with 1 or 2.
+@pytest.mark.parametrize("experts,used,count", [(33, 16, 680), (33, 16, 681), (130, 8, 224), (130, 8, 225),
+                                                (8, 8, 2048), (8, 8, 2049)])
+def test_moe_prefill_router_large_batches(dev, experts, used, count):
+    check_router_order_of_sums(dev, experts, used, count)
+
+
+def check_router_order_of_sums(dev, experts, used, count):
     host = HostLayer(experts, used, biases=True, seed=0x77000160, fill_experts=[])
     rs = np.random.RandomState(experts + count)
     row = O.synth_normal(0x78000160, 0, N, sigma=0.02)

@@ -666,9 +666,12 @@ __global__ __launch_bounds__(256) void router_select_kernel(const float *__restr
 // Router logits of a batch in the reference's own order (matmul_add_f32,
 // tensor.cpp:498-527: sum = bias, then sum = sum + w[c] * x[c] for c = 0..2879,
 // every product and every sum rounded to f32).  Each logit is one chain of 2880
-// dependent adds, 4.3 cycles each (5.6 us), which bounds a batch of up to 512 tokens over 32
-// experts: its chains leave most SIMDs idle, and a wave that forms its own products issues
-// two VALU operations per column where the chain needs one.  So a workgroup takes 4 tokens x
+// dependent adds, 4.3 cycles each (5.6 us).  Two kernels, by the batch's size
+// (launch_router_batch).
+//
+// Up to two workgroups per CU (512 tokens over 64 experts): the chains leave SIMDs idle, and
+// a wave that forms its own products issues two VALU operations per column where the chain
+// needs one.  So a workgroup takes 4 tokens x
 // 16 experts, three waves form the products of a tile of 96 columns, 32 columns each, and
 // wave 0 (lane l: token l / 16, expert l % 16) adds the tile before it up in column order.
 // A producer's lane holds columns 4 (l % 8) .. + 3 of experts l / 8 and 8 + l / 8 and of the
@@ -678,9 +681,8 @@ __global__ __launch_bounds__(256) void router_select_kernel(const float *__restr
 // producer's loads reach five tiles ahead, the summing wave's reads one.  Past the batch or
 // the experts, a lane reads a stand-in row and stores nothing.
 // Barrier t ends tile t's products; every wave arrives at kRcTiles of them.
-// A launch, against one wave per 64 tokens of an expert that formed its own products: 1 to
-// 256 tokens over 32 experts 24 to 12 us, 512 26 to 14, 1000 54 to 23; over 128 experts 40
-// tokens 24 to 12, 256 50 to 20, 512 95 to 40 (two rounds of two workgroups per CU).
+// A launch, against router_lanes_batch_kernel: over 32 experts 512 tokens 16.7 us (25.4),
+// 1024 22.0 (23.6); over 128 experts 64 tokens 12.1 (23.8), 128 13.3 (25.4), 256 20.1 (24.1).
 constexpr int kRcTokens = 4, kRcExperts = 16;
 constexpr int kRcProducers = 3, kRcCols = 32;              // columns per producer and tile
 constexpr int kRcTileCols = kRcProducers * kRcCols;        // 96
@@ -799,6 +801,168 @@ router_chain_batch_kernel(const float *__restrict__ weight, const float *__restr
     }
     if (token < count && expert < experts) {
         logits[size_t(token) * experts + expert] = sum;
+    }
+}
+
+// The same logits for a batch whose chains fill the chip: no product passes through LDS.  Lane
+// l of wave w runs token blockIdx.x * 64 + l against expert blockIdx.y * 4 + w.  The
+// workgroup's 64 token rows are staged a tile of kRlCols columns at a time into one of two
+// LDS buffers, the next tile's loads in flight while the waves run the current one (one
+// barrier per tile); a lane reads its token's columns 16 bytes at a time.  The expert's
+// weights reach the products through DPP: for each 64-column group g of the tile, lane l
+// holds columns 64 g + 4 (l % 16) .. + 3 (each 16-lane row the same), and the product of
+// column 64 g + 4 j + i takes component i from lane j of its row (row_newbcast), so the
+// broadcast costs no instruction.  One wave per SIMD: a wave's two VALU operations per column
+// (product, sum) are the chain's issue rate, 25 us a round of one workgroup per CU.  Logits go
+// to logits[token * experts + expert]; past the batch or the experts, a lane reads a stand-in
+// row and stores nothing.
+// A launch, against router_chain_batch_kernel: over 128 experts 272 tokens 25.5 us (30.2), 400
+// 27.0 (38.8), 512 27.1 (41.4), 576 48.4 (52.2), 1024 48.7 (75.7), 2048 101 (150); over 32
+// experts 1100 tokens 25.9 (31.6), 2048 29.2 (41.6), 2304 50.4 (48.6), 3072 49.8 (59.1).
+constexpr int kRlTokens = 64, kRlWaves = 4;
+constexpr int kRlGroups = 3;                 // 64-column groups per tile
+constexpr int kRlCols = 64 * kRlGroups;      // 15 tiles
+constexpr int kRlStride = kRlCols + 4;       // floats; stride / 4 odd: the lanes' b128 reads miss each other's banks
+constexpr int kRlQuads = kRlCols / 4;
+static_assert(kRouterCols % kRlCols == 0 && (kRlStride / 4) % 2 == 1, "whole tiles, conflict-free rows");
+
+// lane j of the caller's 16-lane row (row_newbcast:j)
+template <int J>
+__device__ __forceinline__ float row_bcast(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + J, 0xf, 0xf, true));
+}
+
+__global__ __launch_bounds__(64 * kRlWaves) void router_lanes_batch_kernel(
+    const float *__restrict__ weight, const float *__restrict__ bias, const float *__restrict__ x, uint32_t x_stride,
+    uint32_t count, uint32_t experts, float *__restrict__ logits) {
+    constexpr int kTiles = kRouterCols / kRlCols;
+    constexpr int kPer = kRlTokens * kRlQuads / (64 * kRlWaves);  // token pieces (16 bytes) per thread and tile
+    constexpr int kChunk = 4;                                     // float4 of x per LDS read batch
+    constexpr int kChunks = kRlQuads / kChunk;
+    static_assert(kRlTokens * kRlQuads % (64 * kRlWaves) == 0 && 16 % kChunk == 0,
+                  "whole pieces, chunks within a group");
+    constexpr int kStaged = (kPer + kChunks - 1) / kChunks;  // staged pieces per chunk
+    static_assert(kTiles % 2 == 1, "tile pairs, then the last tile");
+    // a native vector (not HIP's float4 struct), so the staged pieces stay in registers
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    __shared__ __attribute__((aligned(16))) float xs[2][kRlTokens * kRlStride];
+    const uint32_t t = threadIdx.x, lane = t % 64;
+    const uint32_t wave = uint32_t(__builtin_amdgcn_readfirstlane(int(t / 64)));
+    const uint32_t token0 = blockIdx.x * kRlTokens;
+    const uint32_t last = count - 1 - token0;  // the grid covers the batch: token0 < count
+    const uint32_t expert = blockIdx.y * kRlWaves + wave;
+    const f4 *wsrc =
+        reinterpret_cast<const f4 *>(weight + size_t(min(expert, experts - 1)) * kRouterCols) + lane % 16;
+    // token piece i of a tile: token (t + 64 kRlWaves i) / kRlQuads (clamped to the batch),
+    // float4 (t + 64 kRlWaves i) % kRlQuads
+    const float *xg = x + size_t(token0) * x_stride;
+    uint32_t src[kPer], dst[kPer];  // float offsets from xg, from the LDS buffer
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+        const uint32_t p = t + 64u * kRlWaves * uint32_t(i);
+        src[i] = min(p / kRlQuads, last) * x_stride + 4 * (p % kRlQuads);
+        dst[i] = (p / kRlQuads) * kRlStride + 4 * (p % kRlQuads);
+    }
+    // Two register sets of a tile's token pieces: tile t + 1 is stored from set
+    // (t + 1) % 2 at tile t, which then loads tile t + 3, so a tile's loads have two
+    // tiles' time to land.  The weights are loaded a tile ahead.
+    f4 ra[kPer], rb[kPer], wt[kRlGroups], wn[kRlGroups];
+    auto load = [&](f4(&r)[kPer], int tile) __attribute__((always_inline)) {
+        const float *xt = xg + min(tile, kTiles - 1) * kRlCols;  // past the last tile: a re-read, unused
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            r[i] = *reinterpret_cast<const f4 *>(xt + src[i]);
+        }
+    };
+    auto load_w = [&](f4(&w)[kRlGroups], int tile) __attribute__((always_inline)) {
+        tile = min(tile, kTiles - 1);
+#pragma unroll
+        for (int g = 0; g < kRlGroups; ++g) {
+            w[g] = wsrc[tile * kRlQuads + 16 * g];
+        }
+    };
+    auto store = [&](const f4(&r)[kPer], int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            *reinterpret_cast<f4 *>(xs[buf] + dst[i]) = r[i];
+        }
+    };
+    load(ra, 0);
+    load_w(wt, 0);
+    store(ra, 0);
+    load(rb, 1);
+    load(ra, 2);
+    float sum = bias[min(expert, experts - 1)];
+    __syncthreads();
+    // tile `tile` from LDS buffer tile % 2 with the weights in wt; before chunk c,
+    // stage(i) for its kStaged pieces i (a staged piece's store and its next load,
+    // spread over the tile so a wave never waits to issue a burst of loads)
+    auto compute = [&](int buf, auto &&stage) __attribute__((always_inline)) {
+        const f4 *row = reinterpret_cast<const f4 *>(xs[buf] + lane * kRlStride);
+        f4 xa[kChunk], xb[kChunk];
+#pragma unroll
+        for (int q = 0; q < kChunk; ++q) {
+            xa[q] = row[q];
+        }
+        static_for<kChunks>([&](auto cc) __attribute__((always_inline)) {
+            constexpr int c = decltype(cc)::value;
+            f4(&xc)[kChunk] = c % 2 == 0 ? xa : xb;
+            f4(&xn)[kChunk] = c % 2 == 0 ? xb : xa;
+            if constexpr (c + 1 < kChunks) {
+#pragma unroll
+                for (int q = 0; q < kChunk; ++q) {
+                    xn[q] = row[(c + 1) * kChunk + q];
+                }
+            }
+            static_for<kStaged>([&](auto kk) __attribute__((always_inline)) {
+                constexpr int i = c * kStaged + decltype(kk)::value;
+                if constexpr (i < kPer) {
+                    stage(std::integral_constant<int, i>{});
+                }
+            });
+            __builtin_amdgcn_sched_barrier(0);
+            const f4 w = wt[c * kChunk / 16];
+            static_for<kChunk>([&](auto kk) __attribute__((always_inline)) {
+#pragma clang fp contract(off)
+                constexpr int J = (c * kChunk) % 16 + decltype(kk)::value;
+                const f4 xq = xc[decltype(kk)::value];
+                const float p0 = row_bcast<J>(w.x) * xq.x, p1 = row_bcast<J>(w.y) * xq.y;
+                const float p2 = row_bcast<J>(w.z) * xq.z, p3 = row_bcast<J>(w.w) * xq.w;
+                sum = sum + p0;
+                sum = sum + p1;
+                sum = sum + p2;
+                sum = sum + p3;
+            });
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+    // one tile: tile + 1 into LDS buffer (tile + 1) % 2 (last read before the previous
+    // barrier) from the set S holding it, which then loads tile + 3; the weights of
+    // tile + 1 are loaded meanwhile and move to wt after this tile's products
+    auto step = [&](auto s_, int tile) __attribute__((always_inline)) {
+        constexpr int S = decltype(s_)::value;  // (tile + 1) % 2
+        f4(&r)[kPer] = S == 1 ? rb : ra;
+        load_w(wn, tile + 1);
+        const float *xt = xg + min(tile + 3, kTiles - 1) * kRlCols;  // past the last tile: a re-read, unused
+        compute(S ^ 1, [&](auto i_) __attribute__((always_inline)) {
+            constexpr int i = decltype(i_)::value;
+            *reinterpret_cast<f4 *>(xs[S] + dst[i]) = r[i];
+            r[i] = *reinterpret_cast<const f4 *>(xt + src[i]);
+        });
+#pragma unroll
+        for (int g = 0; g < kRlGroups; ++g) {
+            wt[g] = wn[g];
+        }
+        __syncthreads();  // every wave is done with buffer tile % 2 before it is refilled
+    };
+#pragma unroll 1
+    for (int tile = 0; tile + 1 < kTiles; tile += 2) {
+        step(std::integral_constant<int, 1>{}, tile);
+        step(std::integral_constant<int, 0>{}, tile + 1);
+    }
+    compute((kTiles - 1) % 2, [](auto) {});
+    if (lane <= last && expert < experts) {
+        logits[size_t(token0 + lane) * experts + expert] = sum;
     }
 }
 
@@ -1512,9 +1676,17 @@ int launch_router_batch(ttl_ctx *ctx, const ttl_moe_layer &L, const float *x, ui
     // then the selection
     static_assert(sizeof(RouterScratch) >= 4 * kMaxExperts + 4, "a token's scratch holds its logits and its shift");
     float *logits = static_cast<float *>(scratch);
+    // up to two workgroups of router_chain_batch_kernel per CU run at once; a larger batch is
+    // faster with a lane per logit (both kernels' times stand above them; the same bits)
     const dim3 chains((count + kRcTokens - 1) / kRcTokens, (L.experts + kRcExperts - 1) / kRcExperts);
-    router_chain_batch_kernel<<<chains, 64 * (kRcProducers + 1), 0, ctx->stream>>>(
-        L.router_weight, L.router_bias, x, L.hidden, count, L.experts, logits);
+    if (uint64_t(chains.x) * chains.y <= 2 * uint64_t(ctx->compute_units)) {
+        router_chain_batch_kernel<<<chains, 64 * (kRcProducers + 1), 0, ctx->stream>>>(
+            L.router_weight, L.router_bias, x, L.hidden, count, L.experts, logits);
+    } else {
+        const dim3 lanes((count + kRlTokens - 1) / kRlTokens, (L.experts + kRlWaves - 1) / kRlWaves);
+        router_lanes_batch_kernel<<<lanes, 64 * kRlWaves, 0, ctx->stream>>>(
+            L.router_weight, L.router_bias, x, L.hidden, count, L.experts, logits);
+    }
     if (shift) {
         router_select_logits_kernel<true>
             <<<count, 64, 0, ctx->stream>>>(logits, L.experts, L.used, indices, weights, x, shift);
