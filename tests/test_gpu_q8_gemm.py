@@ -37,7 +37,7 @@ def oracle_matmul(blocks, bias, rows, cols, x, tokens):
 @pytest.mark.parametrize("cols", [2880, 4096])
 @pytest.mark.parametrize("tokens", [1, 5, 64, 70, 200])
 def test_q8_matmul_matches_oracle(dev, cols, tokens):
-    rows = 176  # 11 row tiles: the last workgroup's waves are partly idle
+    rows = 176  # 11 row tiles: tiles of 1 sub-tile x 1 row tile at every one of these counts
     blocks = O.synth_q8_0(21, cols + tokens, rows * cols // 32)
     x = O.synth_normal(22, cols + tokens, tokens * cols, sigma=1.5).reshape(tokens, cols)
     bias = O.synth_normal(23, cols, rows, sigma=0.1)
@@ -72,13 +72,36 @@ def test_q8_matmul_residual_and_no_bias(dev):
     t.free()
 
 
-# One call per tile shape and K split that the launch picks (on 256 CUs: 1x1, 1x2, 2x2,
-# 2x3, 2x5 on 8 waves; 2x5 on 4; 4x3 and 4x5 on 8 and on 4 waves), with a last row group and
-# a last token group that are partly empty.  Against 64 bits: the planes hold 2^-22 of each
-# value and a row sums at most 4096 products, so 1e-6 relative covers both.
-@pytest.mark.parametrize("rows,cols,tokens", [
+# Calls that reach every tile shape (16-token sub-tiles x 16-row tiles) and K split (waves)
+# that the launch picks on 256 CUs, for both widths, with a last row group and a last token
+# group that are partly empty, and the sizes of the model's own short prompts.
+TILE_CALLS = [
     (2880, 4096, 15), (5104, 2880, 16), (5104, 2880, 31), (2864, 4096, 125), (5104, 2880, 125), (5104, 2880, 289),
-    (2864, 4096, 250), (5104, 2880, 250), (2864, 4096, 509), (5104, 2880, 509), (5104, 2880, 1)])
+    (2864, 4096, 250), (5104, 2880, 250), (2864, 4096, 509), (5104, 2880, 509), (5104, 2880, 1),
+    (2864, 4096, 31), (2864, 4096, 61), (2880, 4096, 77), (2864, 4096, 221), (2864, 4096, 445), (2864, 4096, 605),
+    (2864, 4096, 861), (2864, 2880, 15), (5104, 2880, 61), (5120, 2880, 77), (2864, 2880, 250), (5104, 2880, 445)]
+
+
+def tile_shape(rows, tokens, cus):
+    """The shape with the least rounds x (2 sub-tiles + 1) x (row tiles + 1), the first of equals;
+    its waves."""
+    def cost(shape):
+        groups = -(-(-(-tokens // 16)) // shape[0]) * -(-(-(-rows // 16)) // shape[1])
+        return -(-groups // cus) * (2 * shape[0] + 1) * (shape[1] + 1), groups
+    subs, tiles = min([(1, 1), (1, 2), (2, 2), (2, 3), (2, 5), (4, 3), (4, 5)], key=lambda s: cost(s)[0])
+    return subs, tiles, 4 if subs * tiles > 6 and cost((subs, tiles))[1] > cus else 8
+
+
+def test_q8_matmul_calls_reach_every_tile_shape(dev):
+    shapes = {(1, 1, 8), (1, 2, 8), (2, 2, 8), (2, 3, 8), (2, 5, 8), (2, 5, 4), (4, 3, 8), (4, 3, 4), (4, 5, 8), (4, 5, 4)}
+    assert dev.info()["compute_units"] == 256
+    for width in (2880, 4096):
+        assert {tile_shape(r, n, 256) for r, c, n in TILE_CALLS if c == width} == shapes
+
+
+# Against 64 bits: the planes hold 2^-22 of each value and a row sums at most 4096 products, so
+# 1e-6 relative covers both.
+@pytest.mark.parametrize("rows,cols,tokens", TILE_CALLS)
 def test_q8_matmul_tile_shapes(dev, rows, cols, tokens):
     blocks = O.synth_q8_0(31, cols + tokens, rows * cols // 32)
     x = O.synth_normal(32, cols + tokens, tokens * cols).reshape(tokens, cols)
@@ -168,6 +191,39 @@ def test_q8_matmul_token_magnitudes_and_nonfinite(dev, cols):
         assert not np.all(np.isfinite(ref[[7, 8, 9]]))
         assert_matches_with_nonfinite(got, ref, tokens)
         assert np.array_equal(got[6], bias)  # a zero token: the bias alone
+    finally:
+        for b in (xb, bb, ob):
+            b.free()
+        t.free()
+
+
+# The same tokens first, last and in between in a call whose workgroups take four sub-tiles of
+# tokens and several row tiles (4x3 on 4 waves, 4x5 on 8; the last sub-tile has 13 tokens): a
+# token's shift, infinities and NaN stay its own.  The tokens between them against 64 bits.
+@pytest.mark.parametrize("cols", [2880, 4096])
+@pytest.mark.parametrize("tokens,shape", [(509, (4, 3, 4)), (445, (4, 5, 8))])
+def test_q8_matmul_magnitudes_across_sub_tiles(dev, cols, tokens, shape):
+    rows = 2864
+    assert tile_shape(rows, tokens, dev.info()["compute_units"]) == shape
+    blocks = O.synth_q8_0(35, cols, rows * cols // 32)
+    x = O.synth_normal(36, cols, tokens * cols).reshape(tokens, cols)
+    special = np.concatenate([np.arange(12), 245 + np.arange(12), tokens - 12 + np.arange(12)])
+    x[special] = np.tile(magnitude_rows(37 + cols, 12, cols), (3, 1))
+    bias = O.synth_normal(38, cols, rows, sigma=0.1)
+    t = dev.q8_upload(blocks, rows, cols)
+    xb, bb, ob = dev.upload(x), dev.upload(bias), dev.alloc(tokens * rows * 4)
+    try:
+        dev.matmul_q8_0(t, bb, xb, tokens, None, ob)
+        got = ob.download(np.float32).reshape(tokens, rows)
+        with np.errstate(all="ignore"):
+            ref = oracle_matmul(blocks, bias, rows, cols, x[:12], 12)
+        for first in (0, 245, tokens - 12):
+            assert_matches_with_nonfinite(got[first:first + 12], ref, 12)
+            assert np.array_equal(got[first + 6], bias)
+        rest = np.setdiff1d(np.arange(tokens), special)
+        exact = x[rest].astype(np.float64) @ q8_dense(blocks, rows, cols).T + bias
+        for p, e in zip(rest, exact):
+            assert O.rel_l2(got[p], e) < 1e-6, p
     finally:
         for b in (xb, bb, ob):
             b.free()
