@@ -354,11 +354,11 @@ def test_attention_prefill_chunk_edges(dev, layer_index, first, tokens):
 
 
 # Values the three bf16 planes do not take (K of 2^60 and more, V of 2^100 and more,
-# infinities; a query of 2^60) next to ordinary ones: the chunks that hold them, and no
+# infinities and NaN; a query of 2^60) next to ordinary ones: the chunks that hold them, and no
 # others, run on f32 MFMA.  Finite outputs within the usual bar, the others where the
 # oracle has them.
 @pytest.mark.parametrize("layer_index", [0, 1])
-@pytest.mark.parametrize("kind", ["k_large", "k_inf", "v_large", "v_inf", "q_large"])
+@pytest.mark.parametrize("kind", ["k_large", "k_inf", "k_nan", "v_large", "v_inf", "v_nan", "q_large", "q_inf", "q_nan"])
 def test_attention_prefill_wide_values(dev, layer_index, kind):
     first, tokens = 90, 40
     capacity = first + tokens
@@ -373,8 +373,14 @@ def test_attention_prefill_wide_values(dev, layer_index, kind):
         k2[100, 3, 5] = np.inf
     elif kind == "v_large":
         v2[70, 2] *= np.float32(2.0**101)
+    elif kind == "k_nan":
+        k2[100, 3, 5] = np.nan
     elif kind == "v_inf":
         v2[70, 2, 9] = -np.inf
+    elif kind == "v_nan":
+        v2[100, 2, 9] = np.nan
+    elif kind in ("q_inf", "q_nan"):
+        q2[5, 17, 40] = np.inf if kind == "q_inf" else np.nan
     else:
         q2[5, 17] *= np.float32(2.0**60)
     check_attention_prefill(dev, q, k, v, sinks, layer_index, first, tokens, capacity)
