@@ -93,6 +93,33 @@ def test_selected_matmul_matches_oracle(dev, count):
     w.free()
 
 
+# One expert's slots on full tiles and a tiny or narrow last one, where the shares that the 8
+# XCDs take of each kind round up together: 7 x 15 (9 x 1) workgroups of the one and 15 (1) of
+# the other, more than the grid has without the rows that it adds for this.  A workgroup too
+# few would leave rows as they were.
+@pytest.mark.parametrize("rows,count", [(N, 449), (N, 465), (192, 577), (192, 593)])
+@pytest.mark.parametrize("mxfp8", [False, True])
+def test_selected_matmul_covers_every_tile(dev, rows, count, mxfp8):
+    blocks = O.synth_mxfp4(0x77000002, 17, rows * 90)
+    x = O.synth_normal(0x78000002, 19, count * N).reshape(count, N)
+    w = dev.mxfp4_upload(blocks, rows, N, 1)
+    xb, tb = dev.upload(x), dev.upload(np.arange(count, dtype=np.int32))
+    out = dev.upload(np.full(count * rows, np.nan, np.float32))
+    dev.matmul_mxfp4_selected(w, None, xb, N, count, tb, count, out, 0, mxfp8=mxfp8)
+    got = out.download(np.float32).reshape(count, rows)
+    assert np.all(np.isfinite(got))
+    parts = []  # a tile at a time gives the same bits
+    for first in range(0, count, 64):
+        n = min(64, count - first)
+        tb.upload(np.arange(first, first + n, dtype=np.int32))
+        dev.matmul_mxfp4_selected(w, None, xb, N, count, tb, n, out, 0, mxfp8=mxfp8)
+        parts.append(out.download(np.float32).reshape(count, rows)[first:first + n])
+    assert np.array_equal(got.view(np.uint32), np.concatenate(parts).view(np.uint32))
+    for b in (xb, tb, out):
+        b.free()
+    w.free()
+
+
 def run_prefill(dev, layer, x, idx, w, dtype):
     count, used = idx.shape
     if dtype == ttlab_amd.TTL_DTYPE_BF16:
