@@ -379,10 +379,10 @@ __global__ __launch_bounds__(kWinThreads) void attn_window_kernel(const float *_
 // What bounds it: on v_mfma_f32_16x16x4_f32 a chunk's two products of a wave take 256
 // instructions of 32 cycles; six bf16 products take 192 of 16, and the second group puts a
 // second wave on each SIMD, whose softmax and splitting partly overlap the other's MFMAs.
-// Matrix cores about 40% busy, the VALU (splits, softmax, addresses) as much.  512 tokens
-// at 1536: 237 us for a sliding and a full layer on f32 MFMA with one group, 111 us now (on
-// the way: planes 134, scores in units of log 2 125, LDS in fragment order and a barrier
-// per group 113).
+// Of the cycles of a full layer at 1536 the matrix cores are busy 46% and the VALU (splits,
+// softmax, addresses) 45%, of a sliding layer's 24% and 40%.  512 tokens at 1536: 237 us for a
+// sliding and a full layer on f32 MFMA with one group, 112 us now (on the way: planes 134,
+// scores in units of log 2 125, LDS in fragment order and a barrier per group 113).
 constexpr int kPfTokens = 16;
 constexpr int kPfQueries = kPfTokens * kGroup;                   // 128
 constexpr int kPfGroups = 2;                                     // groups of four waves

@@ -681,8 +681,8 @@ __global__ __launch_bounds__(256) void router_select_kernel(const float *__restr
 // producer's loads reach five tiles ahead, the summing wave's reads one.  Past the batch or
 // the experts, a lane reads a stand-in row and stores nothing.
 // Barrier t ends tile t's products; every wave arrives at kRcTiles of them.
-// A launch, against router_lanes_batch_kernel: over 32 experts 512 tokens 16.7 us (25.4),
-// 1024 22.0 (23.6); over 128 experts 64 tokens 12.1 (23.8), 128 13.3 (25.4), 256 20.1 (24.1).
+// A launch, against router_lanes_batch_kernel: over 32 experts 512 tokens 15.2 us (25.2),
+// 1024 22.3 (23.9); over 128 experts 64 tokens 12.0 (23.4), 128 13.6 (24.2), 256 20.2 (25.0).
 constexpr int kRcTokens = 4, kRcExperts = 16;
 constexpr int kRcProducers = 3, kRcCols = 32;              // columns per producer and tile
 constexpr int kRcTileCols = kRcProducers * kRcCols;        // 96
@@ -816,9 +816,9 @@ router_chain_batch_kernel(const float *__restrict__ weight, const float *__restr
 // (product, sum) are the chain's issue rate, 25 us a round of one workgroup per CU.  Logits go
 // to logits[token * experts + expert]; past the batch or the experts, a lane reads a stand-in
 // row and stores nothing.
-// A launch, against router_chain_batch_kernel: over 128 experts 272 tokens 25.5 us (30.2), 400
-// 27.0 (38.8), 512 27.1 (41.4), 576 48.4 (52.2), 1024 48.7 (75.7), 2048 101 (150); over 32
-// experts 1100 tokens 25.9 (31.6), 2048 29.2 (41.6), 2304 50.4 (48.6), 3072 49.8 (59.1).
+// A launch, against router_chain_batch_kernel: over 128 experts 272 tokens 24.7 us (29.1), 400
+// 25.3 (38.7), 512 26.6 (38.9), 576 49.2 (51.8), 1024 53.1 (76.6), 2048 102 (146); over 32
+// experts 1100 tokens 26.0 (31.6), 2048 27.6 (41.5), 2304 47.5 (48.8), 3072 49.5 (59.8).
 constexpr int kRlTokens = 64, kRlWaves = 4;
 constexpr int kRlGroups = 3;                 // 64-column groups per tile
 constexpr int kRlCols = 64 * kRlGroups;      // 15 tiles

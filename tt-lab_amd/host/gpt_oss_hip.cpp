@@ -409,7 +409,8 @@ void HipGptOssModel::validate(int32_t token, size_t position) const {
 void HipGptOssModel::set_position(int32_t token, size_t position) {
     // one launch that carries both words, where two copies each waited for the stream; with
     // the logits copied into page-locked memory a forward call of the 20b model at position
-    // 2047 went from 1355 to 1319 us (the step itself takes 1189)
+    // 2047 went from 1284 to 1253 us (five runs of each in turn: 1275 to 1291, 1238 to 1265; the
+    // step itself takes 1186)
     const uint32_t state[2] = {uint32_t(token), uint32_t(position)};
     check(ttl_set_words(ctx_, reinterpret_cast<uint32_t *>(token_), state, 2), "ttl_set_words");
 }
